@@ -188,6 +188,8 @@ struct snl_engine {
     float *pf_dq = nullptr, *pf_dk = nullptr, *pf_dv = nullptr, *pf_gz = nullptr, *pf_beta = nullptr,
           *pf_decay = nullptr;
     void* pf_frags = nullptr;
+    float* pf_gpart = nullptr;  // slice partials of the prefill GEMM (the largest matrix's)
+    size_t pf_gpart_n = 0;
     float* pf_apart = nullptr;  // attention key-part partials (contexts past one part)
     int pf_parts = 1;
     int pf_pos0 = 0;            // cache position of the current prefill pass's row 0
@@ -357,6 +359,7 @@ struct snl_engine {
             if ((rc = dalloc(&pq, gemm_q_bytes(qt, rows, cols))) || (rc = dalloc(&w.ps, gemm_s_floats(rows, cols))))
                 return rc;
             w.pq = pq;
+            pf_gpart_n = std::max(pf_gpart_n, gemm_part_floats(SNL_PF_M, rows, cols));
             if (launch_panel_pack(qt, rows, cols, gen_tmp_q, gen_tmp_s, w.pq, w.ps, stream))
                 return fail(SNL_EDEVICE, "weight init failed");
         }
@@ -427,6 +430,7 @@ struct snl_engine {
             GemmArgs g{};
             g.wq = w.pq;
             g.ws = w.ps;
+            g.part = pf_gpart;
             g.frags = pf_frags;
             g.xs = pf_xs;
             g.y = y;
@@ -685,7 +689,7 @@ int snl_engine::init() {
             (rc = dalloc(&pf_dk, P * std::max<size_t>(key_dim, 1))) || (rc = dalloc(&pf_dv, P * lin_value_dim + 1)) ||
             (rc = dalloc(&pf_gz, P * lin_value_dim + 1)) || (rc = dalloc(&pf_beta, P * nv)) ||
             (rc = dalloc(&pf_decay, P * nv)) || (rc = dalloc((uint8_t**)&pf_frags, frags_bytes(SNL_PF_M, kmax))) ||
-            (rc = dalloc(&d_pstep, 1)))
+            (rc = dalloc(&pf_gpart, pf_gpart_n + 1)) || (rc = dalloc(&d_pstep, 1)))
             return rc;
         pf_parts = attention_prefill_parts(ctx);
         if (pf_parts > 1 && (rc = dalloc(&pf_apart, P * c.n_heads * pf_parts * (c.head_dim + 2)))) return rc;
@@ -2104,27 +2108,31 @@ int snl_gemm(int quant, const void* wq, const float* ws, const float* x, float* 
     // panel-order weights and the token fragments in staging buffers held under the lock until the
     // call has finished on the stream
     static uint8_t* pq = nullptr;
-    static float *ps = nullptr, *xs = nullptr;
+    static float *ps = nullptr, *xs = nullptr, *part = nullptr;
     static void* fr = nullptr;
-    static size_t cap_q = 0, cap_s = 0, cap_f = 0;
+    static size_t cap_q = 0, cap_s = 0, cap_f = 0, cap_p = 0;
     std::lock_guard<std::mutex> lk(g_kstep_mu);
     const size_t qb = gemm_q_bytes(quant, N, K), sf = gemm_s_floats(N, K), fb = frags_bytes(SNL_PREFILL_M, K);
-    if (qb > cap_q || sf > cap_s || fb > cap_f) {
+    const size_t pf = gemm_part_floats(SNL_PREFILL_M, N, K) + 1;
+    if (qb > cap_q || sf > cap_s || fb > cap_f || pf > cap_p) {
         if (hipStreamSynchronize(st) != hipSuccess) return SNL_EDEVICE;
         hipFree(pq);
         hipFree(ps);
         hipFree(fr);
         hipFree(xs);
+        hipFree(part);
         pq = nullptr;
-        ps = xs = nullptr;
+        ps = xs = part = nullptr;
         fr = nullptr;
-        cap_q = cap_s = cap_f = 0;
+        cap_q = cap_s = cap_f = cap_p = 0;
         if (hipMalloc((void**)&pq, qb) != hipSuccess || hipMalloc((void**)&ps, sf * 4) != hipSuccess ||
-            hipMalloc(&fr, fb) != hipSuccess || hipMalloc((void**)&xs, SNL_PREFILL_M * 4) != hipSuccess)
+            hipMalloc(&fr, fb) != hipSuccess || hipMalloc((void**)&xs, SNL_PREFILL_M * 4) != hipSuccess ||
+            hipMalloc((void**)&part, pf * 4) != hipSuccess)
             return SNL_ENOMEM;
         cap_q = qb;
         cap_s = sf;
         cap_f = fb;
+        cap_p = pf;
     }
     if (launch_panel_pack(quant, N, K, wq, ws, pq, ps, st)) return SNL_EDEVICE;
     RowsArgs r{};
@@ -2147,6 +2155,7 @@ int snl_gemm(int quant, const void* wq, const float* ws, const float* x, float* 
     g.M = M;
     g.N = N;
     g.K = K;
+    g.part = part;
     if (launch_mgemm(g, quant, st) || hipStreamSynchronize(st) != hipSuccess) return SNL_EDEVICE;
     return SNL_OK;
 }
@@ -2232,7 +2241,7 @@ int snl_gemm_time(int quant, int N, int K, int M, int reps, double* ms_per_launc
     if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return SNL_EDEVICE;
     const size_t n = (size_t)N * K;
     uint8_t *q = nullptr, *pq = nullptr;
-    float *s = nullptr, *ps = nullptr, *x = nullptr, *y = nullptr, *xs = nullptr;
+    float *s = nullptr, *ps = nullptr, *x = nullptr, *y = nullptr, *xs = nullptr, *part = nullptr;
     void* fr = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = SNL_OK;
@@ -2240,8 +2249,8 @@ int snl_gemm_time(int quant, int N, int K, int M, int reps, double* ms_per_launc
         hipMalloc((void**)&pq, gemm_q_bytes(quant, N, K)) != hipSuccess ||
         hipMalloc((void**)&ps, gemm_s_floats(N, K) * 4) != hipSuccess ||
         hipMalloc((void**)&x, (size_t)M * K * 4) != hipSuccess || hipMalloc((void**)&y, (size_t)M * N * 4) != hipSuccess ||
-        hipMalloc(&fr, frags_bytes(M, K)) != hipSuccess || hipMalloc((void**)&xs, (size_t)(M + 15) / 16 * 64) != hipSuccess ||
-        hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
+        hipMalloc(&fr, frags_bytes(M, K)) != hipSuccess || hipMalloc((void**)&xs, (size_t)(M + 31) / 32 * 128) != hipSuccess ||
+        hipMalloc((void**)&part, (gemm_part_floats(M, N, K) + 1) * 4) != hipSuccess || hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
         rc = SNL_ENOMEM;
     } else {
         RowsArgs r{};
@@ -2263,6 +2272,7 @@ int snl_gemm_time(int quant, int N, int K, int M, int reps, double* ms_per_launc
         g.M = M;
         g.N = N;
         g.K = K;
+        g.part = part;
         float ms = 0.0f;
         if (launch_gen_matrix(0x5EEDull, N, K, 0.02f, quant, q, s, st) ||
             launch_gen_vector(0x5EEEull, (int64_t)M * K, 0, 1.0f, 0, 0, x, st) ||
@@ -2277,7 +2287,7 @@ int snl_gemm_time(int quant, int N, int K, int M, int reps, double* ms_per_launc
         if (!rc) *ms_per_launch = (double)ms / reps;
     }
     (void)hipStreamSynchronize(st);
-    for (void* p : {(void*)q, (void*)s, (void*)pq, (void*)ps, (void*)x, (void*)y, fr, (void*)xs}) (void)hipFree(p);
+    for (void* p : {(void*)q, (void*)s, (void*)pq, (void*)ps, (void*)x, (void*)y, fr, (void*)xs, (void*)part}) (void)hipFree(p);
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     (void)hipStreamDestroy(st);

@@ -89,7 +89,7 @@ struct RowsArgs {
     float eps;
     int perm4;           // 1: element order of the Q4 nibble dequant
     void* frags;         // out: frags_bytes(M, K)
-    float* xs;           // out: per-token scale [roundup(M, 16)]
+    float* xs;           // out: per-token scale [roundup(M, 32)]
 };
 struct GemmArgs {
     const void* wq;      // panel-order quants
@@ -99,10 +99,14 @@ struct GemmArgs {
     float* y;            // y[m * y_stride + n_off + n]
     int y_stride, n_off;
     int M, N, K;
+    float* part;         // scratch of gemm_part_floats(M, N, K) floats; null: slices are not split over blocks
 };
 size_t gemm_q_bytes(int quant, int N, int K);
 size_t gemm_s_floats(int N, int K);
 size_t frags_bytes(int M, int K);
+// slices of K, a rule on the matrix's shape alone; *slice_st: 64-element stages per slice
+int gemm_slices(int N, int K, int* slice_st);
+size_t gemm_part_floats(int M, int N, int K);
 // reference layout (q [N, K] Q8 / [N, K/2] Q4, s [N, K/32]) -> panel order
 int launch_panel_pack(int quant, int N, int K, const void* q, const float* s, void* qp, float* sp, hipStream_t st);
 int launch_rows_to_frags(const RowsArgs& a, hipStream_t s);

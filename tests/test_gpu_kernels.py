@@ -100,6 +100,35 @@ def test_gemm_rows_independent_of_m(torch_cuda, K, oracle, quant):
         assert np.array_equal(ys.cpu().numpy(), full[lo:hi])
 
 
+@pytest.mark.parametrize("quant", [0, 1])
+@pytest.mark.parametrize("n,k,rows", [
+    (24576, 256, (512, 448, 1, 32)),     # whole rounds of the widest blocks plus narrower ones; 32-row blocks
+    (12352, 128, (512, 97, 33)),         # one round of the widest; ragged last panels
+    (8200, 384, (129, 128, 65, 64)),     # 128 x 128 and 64 x 128 blocks
+    (5760, 1152, (193, 129, 128, 5)),    # two slices, the most panels that have any
+    (4096, 1664, (512, 193, 192, 31)),   # slices of 5, 5 and 3: run by one block, and split over blocks
+    (13, 512, (65, 2)), (256, 768, (300,)), (136, 4096, (512, 40, 3))])
+def test_gemm_block_shapes(torch_cuda, K, oracle, quant, n, k, rows):
+    """Every block shape and slice form of the prefill GEMM, at the edges of their ranges: against
+    float64 products (1e-5 of the sum of |terms|: 32-bit sums of up to 52 exact block results), and
+    bitwise the same rows in all of them."""
+    torch = torch_cuda
+    print(f"gemm shapes quant={quant} n={n} k={k} rows={rows}", flush=True)
+    q, s, x = _gemv_case(oracle, quant, n, k, rows[0], seed=3 * n + k)
+    dq, ds, dx = _dev(torch, q), _dev(torch, s), _dev(torch, x)
+    deq = oracle.dequant(q, s, quant, k).astype(np.float64)
+    exact, scale = x.astype(np.float64) @ deq.T, np.abs(x.astype(np.float64)) @ np.abs(deq).T
+    first = None
+    for m in rows:
+        y = torch.full((m, n + 3), -7.0, dtype=torch.float32, device="cuda")
+        K.gemm(quant, dq, ds, dx, y, m, n, k, k, n + 3)
+        got = y.cpu().numpy()
+        assert np.all(got[:, n:] == -7.0)
+        assert np.all(np.abs(got[:, :n] - exact[:m]) <= 1e-5 * scale[:m] + 1e-30)
+        first = got if first is None else first
+        assert np.array_equal(got, first[:m])
+
+
 def test_gemm_time_runs(torch_cuda, K):
     """The isolated GEMM timing used for the long-context roofline returns a positive mean."""
     for quant in (0, 1):
