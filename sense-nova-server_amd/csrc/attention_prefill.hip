@@ -6,8 +6,8 @@
 // cache at the token's cache position.
 //
 // attend: block (kv head, 16 queries, key part), wave w = query head 4*kv + w of the GQA group;
-// the block streams its part of the keys [0, last query's position] (4096 keys per part) in steps
-// of 32 through LDS (K rows and V rows, each staged with 16-byte copies; the V^T fragments come
+// the block streams its part of the keys [0, last query's position] (128 to 4096 keys, part_keys) in
+// steps of 32 through LDS (K rows and V rows, each staged with 16-byte copies; the V^T fragments come
 // back from the V rows through the transposing LDS read, two 8-byte reads per fragment),
 // shared by the group's 4 heads.
 //   scores  S^T = K Q^T on v_mfma_f32_16x16x32_f16: A = 16 keys x 32 dims of K (exact f16),
@@ -22,6 +22,8 @@
 // combine; with several, each part leaves (unnormalised output, running max, sum) and
 // pf_combine_kernel merges the parts in order.
 #include <float.h>
+
+#include <algorithm>
 #include <hip/hip_fp16.h>
 
 #include "common.h"
@@ -35,7 +37,8 @@ namespace {
 
 constexpr int HD = 256, G = 4;
 constexpr int QTILE = 16, KB = 32;
-constexpr int KPART = 4096;  // keys per part when a long context splits the key range
+constexpr int KPART = 4096, KPART_MIN = 128;  // most and fewest keys of a part
+constexpr int kBlocks = 512;                   // blocks a launch aims at
 constexpr int KROW = HD + 8;  // K tile row (halfs): 528 bytes keeps the 16 rows of a read on distinct banks
 constexpr int VROW = HD + 16;  // V row (halfs): 544 bytes, so the 4 rows of a transposed read hit distinct banks
 
@@ -83,8 +86,8 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(AttnArgs a, const PrefillD
     }
 }
 
-__global__ __launch_bounds__(256) void pf_attend_kernel(AttnArgs a, const PrefillDev* st, int M, float* part,
-                                                        int parts_max) {
+__global__ __launch_bounds__(256, 2) void pf_attend_kernel(AttnArgs a, const PrefillDev* st, int M, float* part,
+                                                        int parts, int kpart) {
     __shared__ __align__(16) _Float16 ks[KB * KROW];
     __shared__ __align__(16) _Float16 vs[KB * VROW];
     const int kh = blockIdx.x, q0 = blockIdx.y * QTILE;
@@ -93,9 +96,9 @@ __global__ __launch_bounds__(256) void pf_attend_kernel(AttnArgs a, const Prefil
     const int pos0 = st->pos0;
     const int qn = min(QTILE, M - q0);
     const int kend = pos0 + q0 + qn;  // keys of the block's last query
-    const int p = blockIdx.z, nparts = (kend + KPART - 1) / KPART;
-    if (p >= nparts) return;
-    const int kfirst = p * KPART, kstop = min(kend, kfirst + KPART);
+    const int p = blockIdx.z;
+    const int kfirst = p * kpart, kstop = min(kend, kfirst + kpart);
+    if (kfirst >= kend) return;
     const int q_dim = a.n_heads * HD, kv_dim = a.n_kv * HD;
     const int j = lane & 15, g = lane >> 4;
     const int mq = q0 + j;
@@ -138,37 +141,33 @@ __global__ __launch_bounds__(256) void pf_attend_kernel(AttnArgs a, const Prefil
     const uint16_t* kc = a.kcache + kh * HD;
     const uint16_t* vc = a.vcache + kh * HD;
 
+    // K and V rows of a step: thread (key t >> 3, 32 dims), the next step's loaded while this one's
+    // values are multiplied
+    uint4 kr[4], vr[4];
+    auto load_rows = [&](int kb) {
+        const int kk = kb + (tid >> 3), seg = tid & 7;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) kr[i] = vr[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (kk < kstop) {
+            const uint4* ksrc = reinterpret_cast<const uint4*>(kc + (size_t)kk * kv_dim + seg * 32);
+            const uint4* vsrc = reinterpret_cast<const uint4*>(vc + (size_t)kk * kv_dim + seg * 32);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) kr[i] = ksrc[i];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) vr[i] = vsrc[i];
+        }
+    };
+    load_rows(kfirst);
     for (int kb = kfirst; kb < kstop; kb += KB) {
         __syncthreads();  // the previous step's tiles are consumed
-        {   // K rows: thread (key t >> 3, 32 dims)
+        {
             const int key = tid >> 3, seg = tid & 7;
-            const int kk = kb + key;
-            uint4 r[4];
+            uint4* kdst = reinterpret_cast<uint4*>(ks + key * KROW + seg * 32);
+            uint4* vdst = reinterpret_cast<uint4*>(vs + key * VROW + seg * 32);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) r[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (kk < kstop) {
-                const uint4* src = reinterpret_cast<const uint4*>(kc + (size_t)kk * kv_dim + seg * 32);
+            for (int i = 0; i < 4; ++i) kdst[i] = kr[i];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) r[i] = src[i];
-            }
-            uint4* dst = reinterpret_cast<uint4*>(ks + key * KROW + seg * 32);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dst[i] = r[i];
-        }
-        {   // V rows, as the K rows: thread (key t >> 3, 32 dims)
-            const int key = tid >> 3, seg = tid & 7;
-            const int kk = kb + key;
-            uint4 r[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) r[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (kk < kstop) {
-                const uint4* src = reinterpret_cast<const uint4*>(vc + (size_t)kk * kv_dim + seg * 32);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) r[i] = src[i];
-            }
-            uint4* dst = reinterpret_cast<uint4*>(vs + key * VROW + seg * 32);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dst[i] = r[i];
+            for (int i = 0; i < 4; ++i) vdst[i] = vr[i];
         }
         __syncthreads();
 
@@ -215,6 +214,7 @@ __global__ __launch_bounds__(256) void pf_attend_kernel(AttnArgs a, const Prefil
         lpart = lpart * factor + psum;
         mrun = mnew;
         // ---- values ----
+        load_rows(kb + KB);
 #pragma unroll
         for (int dt = 0; dt < 16; ++dt) {
             o[dt] = o[dt] * factor;
@@ -235,8 +235,8 @@ __global__ __launch_bounds__(256) void pf_attend_kernel(AttnArgs a, const Prefil
     // ---- normalise, gate, store: lane (query j) holds dims 16dt + 4g + r ----
     const float l = xor_sum<32>(xor_sum<16>(lpart));
     if (!qvalid) return;
-    if (parts_max > 1) {  // this part's unnormalised output, running max and sum for the combine
-        float* pp = part + (((size_t)mq * a.n_heads + hh) * parts_max + p) * (HD + 2);
+    if (parts > 1) {  // this part's unnormalised output, running max and sum for the combine
+        float* pp = part + (((size_t)mq * a.n_heads + hh) * parts + p) * (HD + 2);
 #pragma unroll
         for (int dt = 0; dt < 16; ++dt)
 #pragma unroll
@@ -261,11 +261,11 @@ __global__ __launch_bounds__(256) void pf_attend_kernel(AttnArgs a, const Prefil
 // Merge the key parts of one (query, head): block (head, query), thread = dim.  Parts are added
 // in order with weights e^(m_p - max); then the division by the softmax sum and the sigmoid gate.
 __global__ __launch_bounds__(HD) void pf_combine_kernel(AttnArgs a, const PrefillDev* st, int M, const float* part,
-                                                        int parts_max) {
+                                                        int parts, int kpart) {
     const int hh = blockIdx.x, m = blockIdx.y, d = threadIdx.x;
     const int q0 = m / QTILE * QTILE, qn = min(QTILE, M - q0);
-    const int nparts = (st->pos0 + q0 + qn + KPART - 1) / KPART;
-    const float* pp = part + ((size_t)m * a.n_heads + hh) * parts_max * (HD + 2);
+    const int nparts = (st->pos0 + q0 + qn + kpart - 1) / kpart;
+    const float* pp = part + ((size_t)m * a.n_heads + hh) * parts * (HD + 2);
     float mx = -1e30f;
     for (int p = 0; p < nparts; ++p) mx = fmaxf(mx, pp[(size_t)p * (HD + 2) + HD]);
     float acc = 0.0f, l = 0.0f;
@@ -281,18 +281,40 @@ __global__ __launch_bounds__(HD) void pf_combine_kernel(AttnArgs a, const Prefil
 
 }  // namespace
 
-int attention_prefill_parts(int ctx) { return (ctx + KPART - 1) / KPART; }
+// Keys per part of a pass over `keys` keys: as many parts as give the chip kBlocks blocks (two fit a
+// CU), of at least KPART_MIN keys, and no part longer than KPART.  A step of 32 keys is a chain of
+// loads, LDS and dependent MFMAs that one block alone takes 3.3 us for, so few blocks of many steps
+// leave the chip idle: 16 heads, 45 rows over 1045 keys 109 us in 12 blocks, 18 + 9 (combine) in 108;
+// 512 rows over 1000 keys 83 us in 128 blocks, 28 + 15 in 512; 512 rows at 12800 keys 382 us in parts
+// of 4096, 192 + 17 in four of 3200 (both also with the next step's rows loaded ahead).
+static int part_keys(int M, int n_kv, int keys) {
+    const int base = n_kv * ((M + QTILE - 1) / QTILE);
+    const int parts = std::max(1, kBlocks / base);
+    return std::min(KPART, std::max(KPART_MIN, ((keys + parts - 1) / parts + KB - 1) / KB * KB));
+}
 
-int launch_attention_prefill(const AttnArgs& a, const PrefillDev* pstep, int M, int keys, float* part, int parts_max,
-                             hipStream_t s) {
+size_t attention_prefill_part_floats(int ctx, int n_heads) {
+    size_t most = 0;
+    for (int m = QTILE; m <= SNL_PF_M; m += QTILE) {
+        const int kp = part_keys(m, n_heads / G, ctx);
+        // a shorter context has shorter parts, so no more of them than kBlocks / base or ctx / KPART
+        const size_t parts = std::max<size_t>((ctx + kp - 1) / kp, std::min(kBlocks / (n_heads / G * (m / QTILE)), ctx / KPART_MIN + 1));
+        most = std::max(most, (size_t)m * n_heads * (parts + 1) * (HD + 2));
+    }
+    return most;
+}
+
+int launch_attention_prefill(const AttnArgs& a, const PrefillDev* pstep, int M, int keys, float* part,
+                             size_t part_floats, hipStream_t s) {
     if (M < 1 || M > SNL_PF_M || a.n_heads != G * a.n_kv || a.rot_dim > HD || a.rot_dim % 2 || !pstep) return -1;
-    const int parts = (keys + KPART - 1) / KPART;  // parts of the pass's longest key range
-    if (parts > 1 && (!part || parts > parts_max)) return -1;
+    const int kpart = part_keys(M, a.n_kv, keys);
+    const int parts = (keys + kpart - 1) / kpart;  // parts of the pass's longest key range
+    if (parts > 1 && (!part || (size_t)M * a.n_heads * parts * (HD + 2) > part_floats)) return -1;
     hipLaunchKernelGGL(pf_prep_kernel, dim3(a.n_heads + 2 * a.n_kv, M), dim3(256), 0, s, a, pstep);
     hipLaunchKernelGGL(pf_attend_kernel, dim3(a.n_kv, (M + QTILE - 1) / QTILE, parts), dim3(256), 0, s, a, pstep, M,
-                       part, parts > 1 ? parts_max : 1);
+                       part, parts, kpart);
     if (parts > 1)
-        hipLaunchKernelGGL(pf_combine_kernel, dim3(a.n_heads, M), dim3(HD), 0, s, a, pstep, M, part, parts_max);
+        hipLaunchKernelGGL(pf_combine_kernel, dim3(a.n_heads, M), dim3(HD), 0, s, a, pstep, M, part, parts, kpart);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

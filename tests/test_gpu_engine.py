@@ -445,6 +445,26 @@ def test_long_prefill_matches_decode_feed(snl_mod):
         e.close()
 
 
+@pytest.mark.parametrize("prefix,rows", [(125, 3), (126, 3), (250, 17), (251, 16), (623, 33), (100, 512)])
+def test_prefill_attention_key_parts(snl_mod, prefix, rows):
+    """A prefill pass over cached keys splits them into parts of at least 128 keys; at the parts'
+    edges it gives the logits of the decode kernels (two tokens a pass) within the tolerance."""
+    cfg = snl_mod.tiny_config()
+    n = prefix + rows
+    e = snl_mod.Engine(cfg, seed=31, quant=0, ctx=n)
+    try:
+        prompt = _prompt(n, cfg.vocab, seed=n)
+        pos = [[i] * 3 for i in range(n)]
+        e.forward(prompt[:prefix], pos[:prefix])
+        lg_a, _ = e.forward(prompt[prefix:], pos[prefix:], logit_rows=2)
+        e.reset()
+        for i in range(0, n, 2):
+            lg_b, _ = e.forward(prompt[i:i + 2], pos[i:i + 2], logit_rows=len(prompt[i:i + 2]) if i + 2 >= n else 0)
+        assert np.abs(lg_a[-1] - lg_b[-1]).max() / np.abs(lg_b).max() < 1e-3
+    finally:
+        e.close()
+
+
 @pytest.mark.parametrize("n", [512, 1024])
 def test_draft_after_full_prefill_chunk(snl_mod, oracle, n):
     """A prompt whose last prefill pass is a full 512 rows leaves the first draft at hidden row 512;
