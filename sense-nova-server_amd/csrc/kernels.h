@@ -232,11 +232,11 @@ struct DnPrefillArgs {
     float *beta, *decay; // scratch [M][n_v]
     float* out;          // [M, n_v*128] (o * w) * silu(z), before the head factor of the norm
     float* ssq;          // [M, n_v, kDeltaPrefillGroups] partial sums of o^2 per column group
-    float* pairs;        // scratch of dn_pairs_floats(M, n_k): k.k and k.q inside blocks of tokens
+    float* blocks;       // scratch of dn_block_floats(M, n_v): the blocks' state-independent matrices
     int conv_dim, n_k, n_v;
 };
 int launch_deltanet_prefill(const DnPrefillArgs& a, int M, hipStream_t s);
-size_t dn_pairs_floats(int M, int n_k);
+size_t dn_block_floats(int M, int n_v);
 
 // ---------------------------------------------------------------- sampler (sampler.hip)
 // src/sampler.rs:99-106: repetition, presence and frequency penalties on logits[tok[i]] in place

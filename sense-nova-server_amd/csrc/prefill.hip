@@ -4,14 +4,11 @@
 // DeltaNet (src/shaders/linear.wgsl:38-140).  The causal conv, SiLU, q/k L2 normalisation and the
 // per-token gates do not depend on the recurrent state, so they run for every token of the chunk
 // at once (dn_conv_kernel, one block per (token, head)); the conv state then takes the chunk's
-// last three inputs (dn_conv_state_kernel).  The recurrence itself runs token by token in
-// dn_recur_kernel with the decode kernel's per-thread layout (8 rows of one state column): 8
-// blocks of 4 waves per value head, each owning 16 state columns in registers.  The tokens go
-// through the state 4 at a time in the blocked form of the delta rule (dn_pairs_kernel forms the
-// block's k.k and k.q scalars); the sums over a column's 128 rows run as DPP rotations inside
-// 16-lane rows plus two cross-row exchanges.  The
-// tokens' inputs stream through LDS in slices of 16.  The state is updated in place in the
-// current slot (a prefill pass has no checkpoint).
+// last three inputs (dn_conv_state_kernel).  The recurrence itself takes 16 tokens at a time in the
+// blocked form of the delta rule, as f32 matrix products: dn_block_kernel forms each block's
+// state-independent matrices, dn_recur_kernel runs the blocks in order, 8 blocks of 4 waves per value
+// head, each owning 16 state columns in registers.  The state is updated in place in the current slot
+// (a prefill pass has no checkpoint).
 #include "common.h"
 #include "kernels.h"
 
@@ -25,7 +22,8 @@ constexpr int DK = 128, DV = 128;
 // the recurrence: 8 blocks of 16 state columns per value head, 4 waves each (one wave per SIMD
 // on every CU for the 32 value heads of the 9B shape)
 constexpr int kCG = kDeltaPrefillGroups, kCols = DV / kCG;
-constexpr int kThreads = 256, kWaves = kThreads / 64, kRows = 8;
+constexpr int kThreads = 256, kWaves = kThreads / 64;
+static_assert(kCols == 16 && kWaves * 32 == DK, "a wave's rows are two 16 x 16 MFMA tiles");
 
 // x[m, 0:h] = dequant(embed[tokens[m]]), x[m, h:2h] = 0 (src/engine.rs:777-790)
 __global__ __launch_bounds__(256) void pf_embed_kernel(const uint32_t* tokens, const int8_t* eq, const float* es,
@@ -97,41 +95,86 @@ __global__ __launch_bounds__(128) void dn_conv_kernel(DnPrefillArgs a) {
     }
 }
 
-// Blocked recurrence: the chunk's tokens go through the state kBlk at a time.  Inside a block
-// the scalars k_b.k_c (c < b) and k_c.q_b (c <= b) do not depend on the state; they are the same
-// for every state column, so one block per (kBlk tokens, key head) forms them here (128 threads, one
-// channel each; wave sums, the two waves added in order).
-// 4 tokens per block measured best (190 us per 512-row visit token by token; 166 / 159 / 187 us
-// for blocks of 2 / 4 / 8: the triangular scalar work grows as the square of the block)
-constexpr int kBlk = 4, kKK = kBlk * (kBlk - 1) / 2, kPairs = kBlk * kBlk;
-__device__ __forceinline__ int kk_idx(int b, int c) { return b * (b - 1) / 2 + c; }       // c < b
-__device__ __forceinline__ int kq_idx(int c, int b) { return kKK + b * (b + 1) / 2 + c; } // c <= b
+// Blocked recurrence: the chunk's tokens go through the state kBlk = 16 at a time.  With decays g_b,
+// G_b = g_0 ... g_b and P_bc = g_{c+1} ... g_b inside a block, token b sees the state
+// G_b S + sum_{c<b} P_bc k_c u_c^T, so the deltas (linear.wgsl:118-136) solve
+//   u_b + beta_b sum_{c<b} P_bc (k_c . k_b) u_c = beta_b (v_b - G_b S^T k_b),
+// a unit lower triangular system whose inverse T does not depend on the state or on the column:
+//   U = T diag(beta) (V - diag(G) K S),
+//   O = diag(G) Q S + A U with A_bc = P_bc (k_c . q_b), c <= b,
+//   S := G_last S + sum_c P_last,c k_c u_c^T.
+// dn_block_kernel forms T diag(beta), A, G and P_last for every block of the chunk at once, one
+// block of 64 threads per (16 tokens, key head); the recurrence is then matrix products.
+constexpr int kBlk = 16;
+struct DnBlock {  // of one (block, value head)
+    float tb[kBlk][kBlk], a[kBlk][kBlk];
+    float g[kBlk], pl[kBlk];
+};
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(128) void dn_pairs_kernel(DnPrefillArgs a, int M) {
-    __shared__ float red[2][kPairs];
-    const int blk = blockIdx.x, kh = blockIdx.y, tid = threadIdx.x, n_k = a.n_k;
-    float kd[kBlk], qd[kBlk];
+// acc += X Y^T over 16 columns of both: xv / yv hold columns 4g .. 4g + 3 of the lane's row l % 16
+// (v_mfma_f32_16x16x4_f32, the 4 lane groups' g as its K); acc row 4g + i, column l % 16
+__device__ __forceinline__ f32x4_t mfma16(const float4& xv, const float4& yv, f32x4_t acc) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv.x, yv.x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv.y, yv.y, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv.z, yv.z, acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(xv.w, yv.w, acc, 0, 0, 0);
+}
+__device__ __forceinline__ float4 as_float4(f32x4_t v) { return make_float4(v[0], v[1], v[2], v[3]); }
+
+__global__ __launch_bounds__(64) void dn_block_kernel(DnPrefillArgs a, int M) {
+    __shared__ float kk[kBlk][kBlk + 1], kq[kBlk][kBlk + 1], lw[4][kBlk][kBlk + 1];
+    const int blk = blockIdx.x, kh = blockIdx.y, lane = threadIdx.x, n_k = a.n_k, n_v = a.n_v, group = n_v / n_k;
+    const int c = lane & 15, g = lane >> 4;
+    const int t = blk * kBlk + c;
+    const float4* kp = reinterpret_cast<const float4*>(a.k + ((size_t)min(t, M - 1) * n_k + kh) * DK) + g;
+    const float4* qp = reinterpret_cast<const float4*>(a.q + ((size_t)min(t, M - 1) * n_k + kh) * DK) + g;
+    f32x4_t dk = {}, dq = {};
 #pragma unroll
-    for (int b = 0; b < kBlk; ++b) {
-        const int t = blk * kBlk + b;
-        kd[b] = t < M ? a.k[((size_t)t * n_k + kh) * DK + tid] : 0.0f;
-        qd[b] = t < M ? a.q[((size_t)t * n_k + kh) * DK + tid] : 0.0f;
+    for (int s = 0; s < DK / 16; ++s) {
+        const float4 k4 = kp[4 * s], q4 = qp[4 * s];
+        dk = mfma16(k4, k4, dk);
+        dq = mfma16(q4, k4, dq);
     }
-    float v[kPairs];
 #pragma unroll
-    for (int b = 1; b < kBlk; ++b)
-#pragma unroll
-        for (int c = 0; c < b; ++c) v[kk_idx(b, c)] = kd[b] * kd[c];
-#pragma unroll
-    for (int b = 0; b < kBlk; ++b)
-#pragma unroll
-        for (int c = 0; c <= b; ++c) v[kq_idx(c, b)] = kd[c] * qd[b];
-    wave_sum_n(v);
-    if ((tid & 63) == 0)
-#pragma unroll
-        for (int i = 0; i < kPairs; ++i) red[tid >> 6][i] = v[i];
+    for (int i = 0; i < 4; ++i) {
+        kk[4 * g + i][c] = dk[i];  // k_b . k_c
+        kq[4 * g + i][c] = dq[i];  // q_b . k_c
+    }
     __syncthreads();
-    if (tid < kPairs) a.pairs[((size_t)blk * n_k + kh) * kPairs + tid] = red[0][tid] + red[1][tid];
+    // lane group g takes value heads g, g + 4, ... of the key head, lane c column c of its matrices
+    // (tokens past the chunk: decay 1, beta 0, so their columns of T diag(beta) are 0)
+    for (int h0 = 0; h0 < group; h0 += 4) {
+        const bool live = h0 + g < group;
+        const int h = kh * group + min(h0 + g, group - 1);
+        float tcol[kBlk];
+        const float beta_c = t < M ? a.beta[(size_t)t * n_v + h] : 0.0f;
+        const float dec_c = t < M ? a.decay[(size_t)t * n_v + h] : 1.0f;
+        DnBlock* out = reinterpret_cast<DnBlock*>(a.blocks) + (size_t)blk * n_v + h;
+        float p = 1.0f, gp = 1.0f;
+#pragma unroll
+        for (int b = 0; b < kBlk; ++b) {
+            const float gb = __shfl(dec_c, (lane & 48) + b), bb = __shfl(beta_c, (lane & 48) + b);
+            p = b > c ? p * gb : 1.0f;  // P_bc
+            gp = b <= c ? gp * gb : gp;
+            lw[g][b][c] = b > c ? bb * (p * kk[b][c]) : 0.0f;
+            if (live) out->a[b][c] = b >= c ? p * kq[b][c] : 0.0f;
+        }
+        if (live) {
+            out->g[c] = gp;
+            out->pl[c] = p;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < kBlk; ++b) {
+            float v = b == c ? 1.0f : 0.0f;
+#pragma unroll
+            for (int j = 0; j < b; ++j) v = fmaf(-lw[g][b][j], tcol[j], v);
+            tcol[b] = v;
+            if (live) out->tb[b][c] = v * beta_c;
+        }
+        __syncthreads();
+    }
 }
 
 // conv state := the chunk's last three inputs (from the old state when the chunk is shorter)
@@ -149,207 +192,129 @@ __global__ __launch_bounds__(256) void dn_conv_state_kernel(DnPrefillArgs a, int
     for (int i = 0; i < 3; ++i) a.conv_state[(size_t)i * cd + ch] = r[i];
 }
 
-// Sum over the 16 row groups (lane >> 2) of the lanes that share lane & 3: rotations by 4 and 8
-// inside each 16-lane row (DPP), then the two rows of each half and the two halves (permlane
-// swaps).
-__device__ __forceinline__ float rowgroup_sum(float v) {
-    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, false));
-    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false));
-    v = xor_sum<16>(v);
-    return xor_sum<32>(v);
-}
-
-// The recurrence over the chunk (linear.wgsl:118-136), kCG blocks per value head.  The tokens'
-// inputs pass through LDS in slices of kTok tokens, the next slice loaded while this one runs.
-constexpr int kTok = 16;
-struct RecurSlice {
-    float q[kTok][DK], k[kTok][DK];
-    float v[kTok][kCols], gz[kTok][kCols];
-    float beta[kTok], decay[kTok];
-    float pr[kTok / kBlk][kPairs];  // the blocks' k.k / k.q scalars
+// The recurrence over the chunk, kCG blocks of 16 state columns per value head.  Wave w holds rows
+// 32w .. 32w + 31 of the block's columns as two MFMA accumulators (row 4g + i, column l % 16), which
+// are also the B operands of K S and Q S (K index g, one MFMA per i).  Per 16 tokens: each wave's
+// share of K S and Q S, their sum over the waves through LDS, U by every wave, the output by one
+// wave, the state update.  All products run on v_mfma_f32_16x16x4_f32.  A wave reads its own inputs,
+// two blocks ahead of the one computed.
+// What bounds it: the chain through a block (two products, an exchange between the waves and another
+// product, 1.6 us per 16 tokens).  512 tokens of 32 heads take 52 us + 7.5 in dn_block_kernel; on the
+// vector ALUs, 4 tokens at a time with every row sum reduced across lanes, they took 154 + 5.
+struct RecurIn {
+    float4 k[2], q[2];   // token l % 16, rows 32w + 16t + 4g ..
+    float kt[2][4];      // token 4g + i, row 32w + 16t + l % 16
+    float v[4], gz[4];   // token 4g + i, column l % 16
+    float4 tb, a, g, pl; // row l % 16, columns 4g ..; tokens 4g ..
+    float glast;
 };
 
 __global__ __launch_bounds__(kThreads) void dn_recur_kernel(DnPrefillArgs a, int M) {
-    extern __shared__ float ored[];  // [kWaves][M]
-    __shared__ RecurSlice sl[2];
+    __shared__ f32x4_t part[2][2][kWaves][64];  // [block parity][K S, Q S][wave][lane]
     const int h = blockIdx.x / kCG, cg = blockIdx.x % kCG;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c = lane & 3, rg = lane >> 2;
-    const int jl = 4 * wave + c, j = cg * kCols + jl;
-    const int n_k = a.n_k, n_v = a.n_v, group = n_v / n_k, kh = h / group;
-    const size_t hoff = (size_t)h * DK * DV;
-    float* S = a.state + hoff;
-    float s[kRows];
+    const int c = lane & 15, g = lane >> 4;
+    const int n_k = a.n_k, n_v = a.n_v, kh = h / (n_v / n_k);
+    const int col = cg * kCols + c, r0 = 32 * wave;
+    float* S = a.state + (size_t)h * DK * DV + col;
+    f32x4_t s[2];
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) s[r] = S[(size_t)(kRows * rg + r) * DV + j];
-    const float norm_w = a.lw[(size_t)a.conv_dim * 4 + 2 * n_v + j];
-
-    // slice loader: thread t takes q/k float4s t, t + kThreads, ... (kTok * 2 * DK / 4 = 1024 of
-    // them), then v/gz of the group's columns (one per thread) and the per-token scalars.  Tokens
-    // past the chunk load as k = q = 0, decay 1, beta 0: they leave the state as it is.
-    constexpr int kQK = kTok * 2 * DK / 4 / kThreads;
-    static_assert(kTok * kCols == kThreads, "one v / gz value per thread");
-    static_assert(kTok % kBlk == 0 && kTok / kBlk * kPairs <= kThreads, "a slice's pair scalars, one per thread");
-    float4 rq[kQK];
-    float rv = 0.0f, rb = 0.0f, rp = 0.0f;
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[t][i] = S[(size_t)(r0 + 16 * t + 4 * g + i) * DV];
+    const float norm_w = a.lw[(size_t)a.conv_dim * 4 + 2 * n_v + col];
     const int nblk = (M + kBlk - 1) / kBlk;
-    auto load = [&](int m0) {
+
+    // Tokens past the chunk read the last one's rows: their columns of T diag(beta) are 0, so they
+    // leave the state as it is, and their outputs are not stored.
+    auto load = [&](int blk, RecurIn& d) {
+        if (blk >= nblk) return;
+        const int tc = min(blk * kBlk + c, M - 1);
+        const float4* kp = reinterpret_cast<const float4*>(a.k + ((size_t)tc * n_k + kh) * DK + r0) + g;
+        const float4* qp = reinterpret_cast<const float4*>(a.q + ((size_t)tc * n_k + kh) * DK + r0) + g;
+        const DnBlock* b = reinterpret_cast<const DnBlock*>(a.blocks) + (size_t)blk * n_v + h;
 #pragma unroll
-        for (int u = 0; u < kQK; ++u) {
-            const int f = tid + kThreads * u;  // 0..1023
-            const int which = f >> 9, rem = f & 511, tk = rem >> 5, d4 = rem & 31;
-            const int m = min(m0 + tk, M - 1);
-            const float* src = (which ? a.k : a.q) + ((size_t)m * n_k + kh) * DK;
-            rq[u] = m0 + tk < M ? reinterpret_cast<const float4*>(src)[d4] : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int t = 0; t < 2; ++t) {
+            d.k[t] = kp[4 * t];
+            d.q[t] = qp[4 * t];
         }
-        {   // kTok * kCols values of v, one per thread
-            const int tk = tid / kCols, col = tid % kCols;
-            const int m = min(m0 + tk, M - 1);
-            rv = a.v[((size_t)m * n_v + h) * DV + cg * kCols + col];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int tr = min(blk * kBlk + 4 * g + i, M - 1);
+            const float* kr = a.k + ((size_t)tr * n_k + kh) * DK + r0 + c;
+            d.kt[0][i] = kr[0];
+            d.kt[1][i] = kr[16];
+            d.v[i] = a.v[((size_t)tr * n_v + h) * DV + col];
+            d.gz[i] = a.gz[((size_t)tr * n_v + h) * DV + col];
         }
-        {
-            const int tk = tid & (kTok - 1), m = min(m0 + tk, M - 1);
-            const bool in = m0 + tk < M;
-            rb = tid < kTok ? (in ? a.beta[(size_t)m * n_v + h] : 0.0f)
-               : tid < 2 * kTok ? (in ? a.decay[(size_t)m * n_v + h] : 1.0f) : 0.0f;
-        }
-        {
-            const int bi = m0 / kBlk + tid / kPairs;
-            rp = tid < kTok / kBlk * kPairs && bi < nblk ? a.pairs[((size_t)bi * n_k + kh) * kPairs + tid % kPairs] : 0.0f;
-        }
+        d.tb = reinterpret_cast<const float4*>(b->tb[c])[g];
+        d.a = reinterpret_cast<const float4*>(b->a[c])[g];
+        d.g = reinterpret_cast<const float4*>(b->g)[g];
+        d.pl = reinterpret_cast<const float4*>(b->pl)[g];
+        d.glast = b->g[kBlk - 1];
     };
-    float rg2 = 0.0f;
-    auto load_gz = [&](int m0) {
-        const int tk = tid / kCols, col = tid % kCols;
-        const int m = min(m0 + tk, M - 1);
-        rg2 = a.gz[((size_t)m * n_v + h) * DV + cg * kCols + col];
-    };
-    auto store = [&](RecurSlice& d) {
+    auto step = [&](int blk, const RecurIn& d) {
+        const int par = blk & 1;
+        f32x4_t ks = {}, qs = {};
 #pragma unroll
-        for (int u = 0; u < kQK; ++u) {
-            const int f = tid + kThreads * u;
-            const int which = f >> 9, rem = f & 511, tk = rem >> 5, d4 = rem & 31;
-            reinterpret_cast<float4*>(which ? d.k[tk] : d.q[tk])[d4] = rq[u];
-        }
-        d.v[tid / kCols][tid % kCols] = rv;
-        d.gz[tid / kCols][tid % kCols] = rg2;
-        if (tid < kTok) d.beta[tid] = rb;
-        else if (tid < 2 * kTok) d.decay[tid - kTok] = rb;
-        if (tid < kTok / kBlk * kPairs) d.pr[tid / kPairs][tid % kPairs] = rp;
-    };
-    load(0);
-    load_gz(0);
-    store(sl[0]);
-    __syncthreads();
-    for (int m0 = 0; m0 < M; m0 += kTok) {
-        const int cur = (m0 / kTok) & 1;
-        const bool more = m0 + kTok < M;
-        if (more) {
-            load(m0 + kTok);
-            load_gz(m0 + kTok);
-        }
-        const RecurSlice& d = sl[cur];
-        const int n = min(kTok, M - m0);
-        for (int t0 = 0; t0 < n; t0 += kBlk) {
-            const int nb = min(kBlk, n - t0);
-            // the block's inputs (tokens past the chunk read as k = q = 0, decay 1, beta 0)
-            float kf[kBlk][kRows], qf[kBlk][kRows], g[kBlk], be[kBlk], vj[kBlk], gzj[kBlk];
+        for (int t = 0; t < 2; ++t) ks = mfma16(d.k[t], as_float4(s[t]), ks);
 #pragma unroll
-            for (int b = 0; b < kBlk; ++b) {
-                const int tk = t0 + b;
-                const float4* qp = reinterpret_cast<const float4*>(d.q[tk] + kRows * rg);
-                const float4* kp = reinterpret_cast<const float4*>(d.k[tk] + kRows * rg);
-                const float4 q0 = qp[0], q1 = qp[1], k0 = kp[0], k1 = kp[1];
-                qf[b][0] = q0.x, qf[b][1] = q0.y, qf[b][2] = q0.z, qf[b][3] = q0.w;
-                qf[b][4] = q1.x, qf[b][5] = q1.y, qf[b][6] = q1.z, qf[b][7] = q1.w;
-                kf[b][0] = k0.x, kf[b][1] = k0.y, kf[b][2] = k0.z, kf[b][3] = k0.w;
-                kf[b][4] = k1.x, kf[b][5] = k1.y, kf[b][6] = k1.z, kf[b][7] = k1.w;
-                g[b] = d.decay[tk];
-                be[b] = d.beta[tk];
-                vj[b] = d.v[tk][jl];
-                gzj[b] = d.gz[tk][jl];
-            }
-            // the starting state against the block's keys and queries: column j's 128-row sums
-            float ak[kBlk], aq[kBlk];
+        for (int t = 0; t < 2; ++t) qs = mfma16(d.q[t], as_float4(s[t]), qs);
+        part[par][0][wave][lane] = ks;
+        part[par][1][wave][lane] = qs;
+        // (one barrier a block: the other parity's sums are read before the next one)
+        __syncthreads();
+        f32x4_t z = part[par][0][0][lane];
 #pragma unroll
-            for (int b = 0; b < kBlk; ++b) {
-                ak[b] = 0.0f;
-                aq[b] = 0.0f;
+        for (int w = 1; w < kWaves; ++w) z = z + part[par][0][w][lane];
+        const float gv[4] = {d.g.x, d.g.y, d.g.z, d.g.w}, pl[4] = {d.pl.x, d.pl.y, d.pl.z, d.pl.w};
 #pragma unroll
-                for (int r = 0; r < kRows; ++r) {
-                    ak[b] = fmaf(s[r], kf[b][r], ak[b]);
-                    aq[b] = fmaf(s[r], qf[b][r], aq[b]);
-                }
-            }
+        for (int i = 0; i < 4; ++i) z[i] = d.v[i] - gv[i] * z[i];
+        const f32x4_t u = mfma16(d.tb, as_float4(z), f32x4_t{});
+        f32x4_t pu;
 #pragma unroll
-            for (int b = 0; b < kBlk; ++b) {
-                ak[b] = rowgroup_sum(ak[b]);
-                aq[b] = rowgroup_sum(aq[b]);
-            }
-            // With G_b = g_0 ... g_b and P_bc = g_{c+1} ... g_b, token b sees the state
-            // G_b S + sum_{c<b} P_bc k_c u_c^T, so its delta (linear.wgsl:118-136) is
-            // u_b = (v_b - G_b S^T k_b - sum_{c<b} P_bc (k_c . k_b) u_c) beta_b, its output
-            // o_b = G_b S^T q_b + sum_{c<=b} P_bc (k_c . q_b) u_c, and after the block the state
-            // is G_3 S + sum_c P_3c k_c u_c^T.
-            const float* pr = d.pr[t0 / kBlk];
-            float G[kBlk], u[kBlk];
-            G[0] = g[0];
+        for (int i = 0; i < 4; ++i) pu[i] = pl[i] * u[i];
 #pragma unroll
-            for (int b = 1; b < kBlk; ++b) G[b] = G[b - 1] * g[b];
+        for (int t = 0; t < 2; ++t)
+            s[t] = mfma16(make_float4(d.kt[t][0], d.kt[t][1], d.kt[t][2], d.kt[t][3]), as_float4(pu), s[t] * d.glast);
+        if (wave == (blk & (kWaves - 1))) {  // the outputs: the waves take turns
+            f32x4_t o = part[par][1][0][lane];
 #pragma unroll
-            for (int b = 0; b < kBlk; ++b) {
-                float kvm = G[b] * ak[b], pbc = 1.0f;
+            for (int w = 1; w < kWaves; ++w) o = o + part[par][1][w][lane];
 #pragma unroll
-                for (int c = b - 1; c >= 0; --c) {
-                    pbc = pbc * g[c + 1];
-                    kvm = kvm + pbc * pr[kk_idx(b, c)] * u[c];
-                }
-                u[b] = (vj[b] - kvm) * be[b];
-            }
+            for (int i = 0; i < 4; ++i) o[i] = gv[i] * o[i];
+            o = mfma16(d.a, as_float4(u), o);
 #pragma unroll
-            for (int b = 0; b < kBlk; ++b) {
-                if (b >= nb) break;
-                float o = G[b] * aq[b] + pr[kq_idx(b, b)] * u[b], pbc = 1.0f;
-#pragma unroll
-                for (int c = b - 1; c >= 0; --c) {
-                    pbc = pbc * g[c + 1];
-                    o = o + pbc * pr[kq_idx(c, b)] * u[c];
-                }
-                const int m = m0 + t0 + b;
-                if (rg == 0) a.out[(size_t)m * n_v * DV + h * DV + j] = (o * norm_w) * gzj[b];
-                float q2 = o * o;
+            for (int i = 0; i < 4; ++i) {
+                const int m = blk * kBlk + 4 * g + i;
+                float q2 = o[i] * o[i];
                 q2 = xor_sum<1>(q2);
                 q2 = xor_sum<2>(q2);
-                if (lane == 0) ored[wave * M + m] = q2;
-            }
-            float pu[kBlk];  // P_3c u_c
-            float pc = 1.0f;
-            pu[kBlk - 1] = u[kBlk - 1];
-#pragma unroll
-            for (int c = kBlk - 2; c >= 0; --c) {
-                pc = pc * g[c + 1];
-                pu[c] = pc * u[c];
-            }
-#pragma unroll
-            for (int r = 0; r < kRows; ++r) {
-                float acc = G[kBlk - 1] * s[r];
-#pragma unroll
-                for (int c = 0; c < kBlk; ++c) acc = fmaf(kf[c][r], pu[c], acc);
-                s[r] = acc;
+                q2 = xor_sum<4>(q2);
+                q2 = xor_sum<8>(q2);
+                if (m >= M) continue;
+                a.out[(size_t)m * n_v * DV + h * DV + col] = (o[i] * norm_w) * d.gz[i];
+                if (c == 0) a.ssq[((size_t)m * n_v + h) * kCG + cg] = q2;
             }
         }
-        __syncthreads();  // every wave is done with sl[cur ^ 1]'s previous contents
-        if (more) store(sl[cur ^ 1]);
-        __syncthreads();
+    };
+    RecurIn d0, d1, d2;
+    load(0, d0);
+    load(1, d1);
+    for (int blk = 0; blk < nblk; blk += 3) {
+        load(blk + 2, d2);
+        step(blk, d0);
+        if (blk + 1 >= nblk) break;
+        load(blk + 3, d0);
+        step(blk + 1, d1);
+        if (blk + 2 >= nblk) break;
+        load(blk + 4, d1);
+        step(blk + 2, d2);
     }
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) S[(size_t)(kRows * rg + r) * DV + j] = s[r];
-    for (int m = tid; m < M; m += kThreads) {
-        float t = 0.0f;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) t = t + ored[w * M + m];
-        a.ssq[((size_t)m * n_v + h) * kCG + cg] = t;
-    }
+        for (int i = 0; i < 4; ++i) S[(size_t)(r0 + 16 * t + 4 * g + i) * DV] = s[t][i];
 }
 
 }  // namespace
@@ -367,15 +332,14 @@ int launch_mhc_coef(const float* part, const float* w, int h, int iterations, fl
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-size_t dn_pairs_floats(int M, int n_k) { return (size_t)((M + kBlk - 1) / kBlk) * n_k * kPairs; }
+size_t dn_block_floats(int M, int n_v) { return (size_t)((M + kBlk - 1) / kBlk) * n_v * (sizeof(DnBlock) / sizeof(float)); }
 
 int launch_deltanet_prefill(const DnPrefillArgs& a, int M, hipStream_t s) {
-    if (M < 1 || M > SNL_PF_M || a.n_k < 1 || a.n_v % a.n_k) return -1;
+    if (M < 1 || M > SNL_PF_M || a.n_k < 1 || a.n_v % a.n_k || !a.blocks) return -1;
     hipLaunchKernelGGL(dn_conv_kernel, dim3(M, 2 * a.n_k + a.n_v), dim3(128), 0, s, a);
     hipLaunchKernelGGL(dn_conv_state_kernel, dim3((a.conv_dim + 255) / 256), dim3(256), 0, s, a, M);
-    if (!a.pairs) return -1;
-    hipLaunchKernelGGL(dn_pairs_kernel, dim3((M + kBlk - 1) / kBlk, a.n_k), dim3(128), 0, s, a, M);
-    hipLaunchKernelGGL(dn_recur_kernel, dim3(a.n_v * kCG), dim3(kThreads), (size_t)kWaves * M * 4, s, a, M);
+    hipLaunchKernelGGL(dn_block_kernel, dim3((M + kBlk - 1) / kBlk, a.n_k), dim3(64), 0, s, a, M);
+    hipLaunchKernelGGL(dn_recur_kernel, dim3(a.n_v * kCG), dim3(kThreads), 0, s, a, M);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

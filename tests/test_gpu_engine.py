@@ -465,6 +465,31 @@ def test_prefill_attention_key_parts(snl_mod, prefix, rows):
         e.close()
 
 
+@pytest.mark.parametrize("rows", [3, 15, 16, 17, 32, 33, 49])
+def test_prefill_recurrence_blocks(snl_mod, rows):
+    """The DeltaNet recurrence of a prefill pass takes 16 tokens at a time, the last block part full:
+    its state and convolution state equal the decode kernels' (one token at a time) within the
+    rounding of 32-bit sums over the tokens, from a state that is not zero."""
+    cfg = snl_mod.tiny_config()
+    e = snl_mod.Engine(cfg, seed=37, quant=1, ctx=128)
+    try:
+        prompt = _prompt(40 + rows, cfg.vocab, seed=rows)
+        pos = [[i] * 3 for i in range(40 + rows)]
+        e.forward(prompt[:40], pos[:40])
+        e.snapshot(0)
+        lg_a, _ = e.forward(prompt[40:], pos[40:], logit_rows=1)
+        st_a, cv_a = e.buffer(3), e.buffer(4)
+        e.restore(0, 40)
+        for i in range(40, 40 + rows):
+            lg_b, _ = e.forward(prompt[i:i + 1], pos[i:i + 1], logit_rows=1)
+        st_b, cv_b = e.buffer(3), e.buffer(4)
+        assert np.abs(st_a - st_b).max() / np.abs(st_b).max() < 1e-3
+        assert np.abs(cv_a - cv_b).max() / np.abs(cv_b).max() < 1e-3
+        assert np.abs(lg_a - lg_b).max() / np.abs(lg_b).max() < 1e-3
+    finally:
+        e.close()
+
+
 @pytest.mark.parametrize("n", [512, 1024])
 def test_draft_after_full_prefill_chunk(snl_mod, oracle, n):
     """A prompt whose last prefill pass is a full 512 rows leaves the first draft at hidden row 512;
