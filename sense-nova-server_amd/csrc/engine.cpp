@@ -182,7 +182,7 @@ struct snl_engine {
     float *mx = nullptr, *hn = nullptr, *m_logits = nullptr;
     // chunked prefill: up to SNL_PF_M rows per pass, launched eagerly (prefill.hip, mgemm.hip,
     // attention_prefill.hip)
-    float *pf_x = nullptr, *pf_proj = nullptr, *pf_act = nullptr, *pf_attn = nullptr, *pf_qbuf = nullptr,
+    float *pf_x = nullptr, *pf_proj = nullptr, *pf_attn = nullptr, *pf_qbuf = nullptr,
           *pf_br = nullptr, *pf_xs = nullptr, *pf_part = nullptr, *pf_coef = nullptr, *pf_ssq = nullptr;
     float* pf_blocks = nullptr;  // prefill DeltaNet: the matrices of its 16-token blocks
     float *pf_dq = nullptr, *pf_dk = nullptr, *pf_dv = nullptr, *pf_gz = nullptr, *pf_beta = nullptr,
@@ -418,7 +418,7 @@ struct snl_engine {
             r.mode = mode;
             r.w = nw;
             r.coef = pf_coef;
-            r.h = h;
+            r.h = mode == ROWS_SWIGLU ? w.cols : h;
             r.ssq = pf_ssq;
             r.eps = cfg.eps;
             r.perm4 = w.quant;
@@ -681,7 +681,7 @@ int snl_engine::init() {
         const int nv = std::max(c.lin_v_heads, 1);
         const size_t key_dim = (size_t)c.lin_k_heads * c.lin_k_dim;
         if ((rc = dalloc(&pf_x, P * 2 * h)) || (rc = dalloc(&pf_proj, P * proj_w)) ||
-            (rc = dalloc(&pf_act, P * c.intermediate)) || (rc = dalloc(&pf_attn, P * attn_w)) ||
+            (rc = dalloc(&pf_attn, P * attn_w)) ||
             (rc = dalloc(&pf_qbuf, P * q_dim)) || (rc = dalloc(&pf_br, P * h)) || (rc = dalloc(&pf_xs, P)) ||
             (rc = dalloc(&pf_part, P * 9)) || (rc = dalloc(&pf_coef, P * 8)) ||
             (rc = dalloc(&pf_ssq, P * nv * kDeltaPrefillGroups)) ||
@@ -866,7 +866,7 @@ int snl_engine::record_mtp(int M, int draft) {
 // One prefill pass of M token rows (up to SNL_PF_M) over the execution plan, the same op order as
 // record_forward with the matrix products on the panel GEMM and the per-token work in prefill
 // kernels: branch inputs become GEMM fragments (rows_to_frags), each mHC site computes its router
-// sums and coefficients over all rows, and merges and SwiGLU run as their own launches.
+// sums and coefficients over all rows, and merges run as their own launches.
 int snl_engine::record_prefill(int M, int rows) {
     const snl_config& c = cfg;
     int rc = 0;
@@ -922,8 +922,7 @@ int snl_engine::record_prefill(int M, int rows) {
         if (op("merge", 0.0)) rc |= launch_merge(pf_x, pf_coef, pf_br, h, M, mhc ? 1 : 0, stream);
         if (mhc) rc |= pf_site(L.mhc_ffn.p, M);
         rc |= pf_mat("gemm_gate_up", L.gate_up, pf_x, X2, M, pro, L.post_ln.p, pf_proj, 2 * c.intermediate);
-        if (op("swiglu", 0.0)) rc |= launch_swiglu(pf_proj, pf_act, c.intermediate, M, stream);
-        rc |= pf_mat("gemm_down", L.down, pf_act, c.intermediate, M, ROWS_PLAIN, nullptr, pf_br, h);
+        rc |= pf_mat("gemm_down", L.down, pf_proj, 2 * c.intermediate, M, ROWS_SWIGLU, nullptr, pf_br, h);
         const int mode = !mhc ? 0 : (li + 1 == c.mhc_end ? 2 : 1);
         if (op("merge", 0.0)) rc |= launch_merge(pf_x, pf_coef, pf_br, h, M, mode, stream);
     }
@@ -957,8 +956,7 @@ int snl_engine::record_mtp_prefill(int M, int r0) {
     rc |= pf_mat("gemm_mtp_o", m_o, pf_attn, q_dim, M, ROWS_PLAIN, nullptr, pf_br, h);
     if (op("merge", 0.0)) rc |= launch_merge(pf_x, pf_coef, pf_br, h, M, 0, stream);
     rc |= pf_mat("gemm_mtp_gate_up", m_gate_up, pf_x, X2, M, ROWS_NORM, m_post_ln.p, pf_proj, 2 * c.intermediate);
-    if (op("swiglu", 0.0)) rc |= launch_swiglu(pf_proj, pf_act, c.intermediate, M, stream);
-    rc |= pf_mat("gemm_mtp_down", m_down, pf_act, c.intermediate, M, ROWS_PLAIN, nullptr, pf_br, h);
+    rc |= pf_mat("gemm_mtp_down", m_down, pf_proj, 2 * c.intermediate, M, ROWS_SWIGLU, nullptr, pf_br, h);
     if (op("merge", 0.0)) rc |= launch_merge(pf_x, pf_coef, pf_br, h, M, 0, stream);
     mark("end", 0.0);
     return rc ? SNL_EDEVICE : SNL_OK;

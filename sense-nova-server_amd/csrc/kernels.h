@@ -75,10 +75,11 @@ int gemv_init();
 // ---------------------------------------------------------------- prefill GEMM (mgemm.hip)
 // Token rows -> the GEMM's f16 hi/lo A fragments, with the branch input computed on the way:
 // the rows as they are, RMSNorm(x0) * (1 + w), the mHC pre-mix then that norm (coef[m][0..1]),
-// or the head factor of the DeltaNet gated norm (ssq partials [M][K/128][kDeltaPrefillGroups]).
-enum RowsMode { ROWS_PLAIN = 0, ROWS_NORM = 1, ROWS_NORM_MHC = 2, ROWS_GNORM = 3 };
+// the head factor of the DeltaNet gated norm (ssq partials [M][K/128][kDeltaPrefillGroups]), or SwiGLU
+// of rows [gate | up].
+enum RowsMode { ROWS_PLAIN = 0, ROWS_NORM = 1, ROWS_NORM_MHC = 2, ROWS_GNORM = 3, ROWS_SWIGLU = 4 };
 struct RowsArgs {
-    const float* x;      // token row m at x + m * x_stride (NORM_MHC: stream 1 at +h)
+    const float* x;      // token row m at x + m * x_stride (NORM_MHC: stream 1, SWIGLU: up row at +h)
     int x_stride;
     int M, K;
     int mode;
@@ -150,9 +151,8 @@ int launch_mhc(const float* x, const float* w, float* part, int h, int M, hipStr
 // x[m, h + i] = x[m, i] (merge mode 3, layers.wgsl:146-149)
 int launch_expand(float* x, int h, int M, hipStream_t s);
 
-// Plain merge (modes 0..2) and SwiGLU, for paths that do not fuse them into a GEMV.
+// Plain merge (modes 0..2), for paths that do not fuse it into a GEMV.
 int launch_merge(float* x, const float* coef, const float* br, int h, int M, int mode, hipStream_t s);
-int launch_swiglu(const float* proj, float* act, int inter, int M, hipStream_t s);
 
 // Greedy pick per logits row: first index of the maximum, the maximum and the second largest value.
 struct Pick {

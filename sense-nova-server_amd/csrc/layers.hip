@@ -195,14 +195,6 @@ __global__ __launch_bounds__(256) void merge_kernel(float* x, const float* coef,
     }
 }
 
-__global__ __launch_bounds__(256) void swiglu_kernel(const float* proj, float* act, int inter, int M) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx >= M * inter) return;
-    const int m = idx / inter, i = idx % inter;
-    const float g = proj[(size_t)m * 2 * inter + i], u = proj[(size_t)m * 2 * inter + inter + i];
-    act[idx] = g / (1.0f + expf(-g)) * u;
-}
-
 // ---- greedy pick: (max, first index of max, second largest) ----
 struct Top2 {
     float v1;
@@ -428,11 +420,6 @@ int launch_expand(float* x, int h, int M, hipStream_t s) {
 int launch_merge(float* x, const float* coef, const float* br, int h, int M, int mode, hipStream_t s) {
     if (mode < 0 || mode > 2) return -1;
     hipLaunchKernelGGL(merge_kernel, dim3((M * h + 255) / 256), dim3(256), 0, s, x, coef, br, h, M, mode);
-    return last_error();
-}
-
-int launch_swiglu(const float* proj, float* act, int inter, int M, hipStream_t s) {
-    hipLaunchKernelGGL(swiglu_kernel, dim3((M * inter + 255) / 256), dim3(256), 0, s, proj, act, inter, M);
     return last_error();
 }
 

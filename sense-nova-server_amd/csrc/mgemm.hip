@@ -129,14 +129,18 @@ __device__ __forceinline__ size_t frag_index(int T, int nb, int u, int t) {
 }
 
 // One block per token row: the row's 8-element groups are held in registers (GPT per thread),
-// the branch input is formed (RMSNorm (1 + w) of stream 0 or of the mHC pre-mix, or the DeltaNet
-// head factor, one per group), then the row's largest magnitude sets the power of two and each
+// the branch input is formed (RMSNorm (1 + w) of stream 0 or of the mHC pre-mix, the DeltaNet head
+// factor, one per group, or SwiGLU of a gate and up row), then the row's largest magnitude sets the power of two and each
 // group is written as its hi and lo halves of the MFMA A fragments.
 template <int GPT>
 __global__ __launch_bounds__(kRowThreads) void rows_to_frags_kernel(RowsArgs a) {
     __shared__ float red[4];
     __shared__ float rs[4];
-    const int m = blockIdx.x, tid = threadIdx.x, K = a.K, nb = K / 32, ngr = K / 8;
+    // Block b runs on XCD b % 8; each XCD takes an eighth of the rows in a run, so the 16-byte pieces of
+    // neighbouring rows that share a fragment's cache lines meet in one L2.  (The grid is whole tiles of
+    // 32 rows.)
+    const int m = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int tid = threadIdx.x, K = a.K, nb = K / 32, ngr = K / 8;
     const int T = m >> 5, t = m & 31;
     half8_t* xf = reinterpret_cast<half8_t*>(a.frags);
     if (m >= a.M) {  // padding rows of the last token tile
@@ -172,6 +176,12 @@ __global__ __launch_bounds__(kRowThreads) void rows_to_frags_kernel(RowsArgs a) 
                 const float u8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
                 for (int e = 0; e < 8; ++e) w8[e] = f0 * w8[e] + f1 * u8[e];
+            } else if (a.mode == ROWS_SWIGLU) {  // layers.wgsl:164-175: silu(gate) * up
+                const float4* q = reinterpret_cast<const float4*>(xr + a.h + 8 * u);
+                const float4 q0 = q[0], q1 = q[1];
+                const float u8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) w8[e] = silu(w8[e]) * u8[e];
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
