@@ -2067,14 +2067,20 @@ int snl_gemv(int quant, const void* wq, const float* ws, const float* x, float* 
     g.N = N;
     g.K = K;
     g.epi = GEMV_STORE;
-    // The engine's kernel reads tile order: pack the caller's reference-layout matrix into a
-    // staging buffer first (held under the lock until the call has finished on the stream).
+    // A Q8 matrix is read where it lies (gemv.hip): packing it into the tile order of the engine's kernel
+    // for one product cost more than the product (2 rows, us a call packed / direct: 12352 x 4096 57 /
+    // 33, 24576 x 4096 87 / 38, 1544 x 256 23 / 18).  Q4 keeps the engine's kernel, and with it the
+    // engine's rounding (its -8 x block sum correction, 2e-6 of a result against 1e-7); so do quants that
+    // 16-byte loads cannot read.  Those are packed into a staging buffer, held under the lock until the
+    // call has finished on the stream.  Shapes of the engine's kernel return when their work is done, the
+    // others when it is queued.
     static uint8_t* pq = nullptr;
     static float* ps = nullptr;
     static size_t cap_q = 0, cap_s = 0;
     std::lock_guard<std::mutex> lk(g_kstep_mu);
     PackGeom pg;
-    if (pack_geom(quant, N, K, 0, &pg) && M >= 1 && M <= SNL_MAX_M && mgemv_fits(M, K)) {
+    const bool waits = pack_geom(quant, N, K, 0, &pg) && M >= 1 && M <= SNL_MAX_M && mgemv_fits(M, K);
+    if (waits && (quant != 0 || (uintptr_t)wq % 16)) {
         if (pg.q_bytes > cap_q || pg.s_floats > cap_s) {
             if (hipStreamSynchronize(st) != hipSuccess) return SNL_EDEVICE;
             hipFree(pq);
@@ -2093,7 +2099,7 @@ int snl_gemv(int quant, const void* wq, const float* ws, const float* x, float* 
         g.ws = ps;
     }
     int rc = launch_gemv(g, quant, M, st);
-    if (rc == 0 && g.packed && hipStreamSynchronize(st) != hipSuccess) rc = -2;
+    if (rc == 0 && waits && hipStreamSynchronize(st) != hipSuccess) rc = -2;
     return rc == -1 ? SNL_EARG : (rc ? SNL_EDEVICE : SNL_OK);
 }
 

@@ -14,18 +14,16 @@
 // One x slice read from LDS serves the 4 rows of the group and all M token rows are applied to
 // each weight byte once: the M=2 verify pass reads each weight once.
 //
-// Dequantisation in registers.  Q8: the word is xor-ed with 0x80808080, which turns each int8 q
-// into the unsigned byte q+128; v_cvt_f32_ubyte{0..3} converts one byte per instruction and the
-// bias is removed once per lane slice, sum (q+128) x - 128 sum x.  Q4: the nibbles are masked
-// into bytes and converted the same way, minus 8 sum x.  The 16-element sums of x are staged in
-// LDS with x.
+// Dequantisation in registers: each quant is converted once, exactly, and multiplied with every
+// token row's element; a lane's 16 products are summed before the block scale is applied.
 //
 // Reduction.  Per group each lane holds 4 row partials per token row; a transposed butterfly
 // (xor 32, 16 exchange halves, then xor 8..1 add) leaves lane 16r with row r.  Every token row
 // takes the same instruction sequence whatever M and its index are.
 //
-// This vector-ALU kernel serves kernel-level calls on row-major weights that the matrix-core
-// kernel (mgemv.hip, tile-order weights) does not take: K % 128 != 0, or M = 3..4 at K > 4096.
+// This kernel serves kernel-level calls (snl_gemv), whose weights come row-major: the engine's
+// matrix-core kernel (mgemv.hip) is faster on weights laid out once, but packing a matrix into tile
+// order for a single product moves it three times.
 // It computes the plain product y = W x.
 #include "common.h"
 #include "kernels.h"
@@ -58,34 +56,21 @@ __device__ __forceinline__ void load_frag(const GemvArgs& a, int row, int k, uin
         }
         sc = a.ws[(size_t)row * (a.K >> 5) + (k >> 5)];
     } else {
-        w[0] = w[1] = w[2] = w[3] = QT == 0 ? 0x80808080u : 0x88888888u;
+        w[0] = w[1] = w[2] = w[3] = QT == 0 ? 0u : 0x88888888u;
         sc = 0.0f;
     }
 }
 
-// sum over the lane's 16 elements of (biased byte value) * x for one token row
+// the lane's 16 quants as exact f32 (Q8: signed bytes; Q4: nibble - 8, as the signed 4 bits of nibble ^ 8)
 template <int QT>
-__device__ __forceinline__ float dot16(const uint32_t (&w)[4], const float (&x)[16]) {
-    float p = 0.0f;
+__device__ __forceinline__ void quants16(const uint32_t (&w)[4], float (&q)[16]) {
     if constexpr (QT == 0) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t u = w[j] ^ 0x80808080u;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) p = fmaf((float)((u >> (8 * b)) & 0xFFu), x[4 * j + b], p);
-        }
+        for (int j = 0; j < 16; ++j) q[j] = (float)(int8_t)(w[j / 4] >> (8 * (j % 4)));
     } else {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t lo = w[j] & 0x0F0F0F0Fu, hi = (w[j] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                p = fmaf((float)((lo >> (8 * b)) & 0xFFu), x[8 * j + 2 * b], p);
-                p = fmaf((float)((hi >> (8 * b)) & 0xFFu), x[8 * j + 2 * b + 1], p);
-            }
-        }
+        for (int j = 0; j < 16; ++j) q[j] = (float)((int)((w[j / 8] ^ 0x88888888u) << (28 - 4 * (j % 8))) >> 28);
     }
-    return p;
 }
 
 // LDS layout of a staged token row: per 1024-element chunk, float4 v (0..3) of lane l sits at
@@ -98,11 +83,10 @@ __device__ __forceinline__ int lds_f4(int k4) {  // k4 = k / 4
 template <int QT, int M>
 __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a, int G) {
     extern __shared__ float4 lds4[];
-    const int K = a.K, K4 = K >> 2, K16 = K >> 4;
+    const int K = a.K, K4 = K >> 2;
     const int nchunks = (K + kChunk - 1) / kChunk;
     const int K4p = nchunks * (kChunk / 4);                         // staged row length, whole chunks
     float4* xs4 = lds4;                                             // [M][K4p] staged rows (permuted)
-    float* sxs = reinterpret_cast<float*>(lds4 + (size_t)M * K4p);  // [M][K/16] 16-element sums
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int blk = blockIdx.x;
     const int steps = G * nchunks;
@@ -121,25 +105,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a, int G) {
         for (int k4 = tid; k4 < K4; k4 += kThreads) xs4[m * K4p + lds_f4(k4)] = xr[k4];
     }
     __syncthreads();
-    // 16-element sums for the dequantisation bias
-#pragma unroll
-    for (int m = 0; m < M; ++m)
-        for (int j = tid; j < K16; j += kThreads) {
-            float s = 0.0f;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float4 t = xs4[m * K4p + lds_f4(4 * j + v)];
-                s = s + t.x;
-                s = s + t.y;
-                s = s + t.z;
-                s = s + t.w;
-            }
-            sxs[m * K16 + j] = s;
-        }
-    __syncthreads();
-
     // ---- streaming main loop ----
-    const float bias = QT == 0 ? 128.0f : 8.0f;
     float acc[4][M];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -156,22 +122,27 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a, int G) {
         }
         const int k = c * kChunk + lane * 16;
         if (k < K) {
+            float xv[M][16];
 #pragma unroll
-            for (int m = 0; m < M; ++m) {
-                float xv[16];
+            for (int m = 0; m < M; ++m)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float4 t = xs4[m * K4p + (c << 8) + (v << 6) + lane];
-                    xv[4 * v] = t.x;
-                    xv[4 * v + 1] = t.y;
-                    xv[4 * v + 2] = t.z;
-                    xv[4 * v + 3] = t.w;
+                    xv[m][4 * v] = t.x;
+                    xv[m][4 * v + 1] = t.y;
+                    xv[m][4 * v + 2] = t.z;
+                    xv[m][4 * v + 3] = t.w;
                 }
-                const float sx = sxs[m * K16 + (k >> 4)];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float p = dot16<QT>(wc[r], xv);
-                    acc[r][m] = fmaf(scc[r], fmaf(-bias, sx, p), acc[r][m]);
+            for (int r = 0; r < 4; ++r) {
+                float q[16];
+                quants16<QT>(wc[r], q);
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    float p = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) p = fmaf(q[e], xv[m][e], p);
+                    acc[r][m] = fmaf(scc[r], p, acc[r][m]);
                 }
             }
         }
@@ -237,7 +208,7 @@ int groups_for(int N) {
 }  // namespace
 
 int gemv_init() {
-    const int bytes = kLdsFloats * 4 + kLdsFloats / 16 * 4;
+    const int bytes = kLdsFloats * 4;
     for (int q = 0; q < 2; ++q)
         for (int M = 1; M <= SNL_MAX_M; ++M) {
             KernelFn f = pick(q, M);
@@ -267,7 +238,7 @@ int launch_gemv(const GemvArgs& a, int quant, int M, hipStream_t s) {
     if (!f) return -1;
     const int G = groups_for(a.N);
     dim3 grid((a.N + 16 * G - 1) / (16 * G));
-    const size_t lds = (size_t)M * K4p * 16 + (size_t)M * (a.K / 16) * 4;
+    const size_t lds = (size_t)M * K4p * 16;
     hipLaunchKernelGGL(f, grid, dim3(kThreads), lds, s, a, G);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }

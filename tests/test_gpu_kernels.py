@@ -59,6 +59,36 @@ def test_gemv_matches_oracle(torch_cuda, K, oracle, quant, n, k, m):
     assert np.all(np.abs(got - exact) <= 1e-5 * scale + 1e-7)
 
 
+@pytest.mark.parametrize("quant,n,k", [(0, 12352, 4096), (0, 13, 128), (0, 16411, 1152), (0, 65537, 256), (0, 21, 1056),
+                                       (1, 21, 1056), (1, 40, 32)])
+def test_gemv_row_major(torch_cuda, K, oracle, quant, n, k):
+    """Weights read where they lie, at the edges of the row groups and K chunks, and a Q8 matrix that
+    16-byte loads cannot read: float64 products within 2e-6 of the sum of |terms| (at most 16 + 8 + 6
+    roundings of 6e-8 on a term), bitwise the same row in calls of 1 and 2 rows."""
+    torch = torch_cuda
+    print(f"gemv row-major quant={quant} n={n} k={k}", flush=True)
+    q, s, x = _gemv_case(oracle, quant, n, k, 2, seed=n + k)
+    deq = oracle.dequant(q, s, quant, k).astype(np.float64)
+    exact, scale = x.astype(np.float64) @ deq.T, np.abs(x.astype(np.float64)) @ np.abs(deq).T
+    flat = np.ascontiguousarray(q).view(np.uint8).ravel()
+    off = torch.empty(flat.size + 16, dtype=torch.uint8, device="cuda")
+    off[4:4 + flat.size] = torch.from_numpy(flat.copy()).cuda()
+    ds, dx = _dev(torch, s), _dev(torch, x)
+    for dq in (_dev(torch, q), off[4:] if k % 128 == 0 else None):
+        if dq is None:
+            continue
+        y = torch.full((2, n + 1), -7.0, dtype=torch.float32, device="cuda")
+        K.gemv(quant, dq, ds, dx, y, 2, n, k, k, n + 1)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        assert np.all(got[:, n] == -7.0)
+        assert np.all(np.abs(got[:, :n] - exact) <= 2e-6 * scale)
+        y1 = torch.zeros((1, n), dtype=torch.float32, device="cuda")
+        K.gemv(quant, dq, ds, dx[1:], y1, 1, n, k, k, n)
+        torch.cuda.synchronize()
+        assert np.array_equal(y1.cpu().numpy()[0], got[1, :n])
+
+
 @pytest.mark.parametrize("quant", [0, 1])
 @pytest.mark.parametrize("n,k,m", [(96, 1024, 3), (4096, 4096, 512), (1544, 256, 37), (12352, 4096, 130),
                                    (4096, 12288, 64), (24576, 4096, 17)])
