@@ -2045,9 +2045,7 @@ static StepDev* g_kstep = nullptr;
 
 static StepDev* kernel_step(const StepDev& h, hipStream_t s) {
     if (!g_kstep && hipMalloc((void**)&g_kstep, sizeof(StepDev)) != hipSuccess) return nullptr;
-    if (hipMemcpyAsync(g_kstep, &h, sizeof(StepDev), hipMemcpyHostToDevice, s) != hipSuccess) return nullptr;
-    if (hipStreamSynchronize(s) != hipSuccess) return nullptr;
-    return g_kstep;
+    return launch_put_step(h, g_kstep, s) ? nullptr : g_kstep;
 }
 
 int snl_gemv(int quant, const void* wq, const float* ws, const float* x, float* y, int M, int N, int K, int x_stride,
@@ -2339,12 +2337,16 @@ int snl_deltanet(const float* proj, int proj_stride, const float* lw, float* con
         hipFree(g_ssq);
         g_ssq = nullptr;
         g_ssq_n = 0;
-        if (hipMalloc((void**)&g_ssq, nss * sizeof(float)) != hipSuccess) return SNL_ENOMEM;
+        if (hipMalloc((void**)&g_ssq, nss * sizeof(float)) != hipSuccess) {
+            (void)hipStreamSynchronize(s);
+            return SNL_ENOMEM;
+        }
         g_ssq_n = nss;
     }
     a.ssq = g_ssq;
-    if (launch_deltanet(a, M, s) || launch_deltanet_norm(a, M, s)) return SNL_EDEVICE;
-    return hipStreamSynchronize(s) == hipSuccess ? SNL_OK : SNL_EDEVICE;
+    // the record and the scratch are free again when the lock is: also on an error, the call waits
+    const int rc = launch_deltanet(a, M, s) || launch_deltanet_norm(a, M, s);
+    return hipStreamSynchronize(s) == hipSuccess && !rc ? SNL_OK : SNL_EDEVICE;
 }
 
 int snl_attention(const float* proj, int proj_stride, float* qbuf, uint16_t* kcache, uint16_t* vcache,
@@ -2383,9 +2385,10 @@ int snl_attention(const float* proj, int proj_stride, float* qbuf, uint16_t* kca
     a.mrope = ((uint32_t)(3 * mrope_section[1]) << 16) | (uint32_t)(3 * mrope_section[2]);
     a.ctx = ctx;
     a.step = d;
-    int rc = launch_attention(a, M, s);
+    const int rc = launch_attention(a, M, s);
+    const hipError_t se = hipStreamSynchronize(s);  // (also on an error: the record is free when the lock is)
     if (rc) return rc == -1 ? SNL_EARG : SNL_EDEVICE;
-    return hipStreamSynchronize(s) == hipSuccess ? SNL_OK : SNL_EDEVICE;
+    return se == hipSuccess ? SNL_OK : SNL_EDEVICE;
 }
 
 int snl_pick_rows(const float* logits, int V, int rows, snl_pick* picks_out, void* stream) {

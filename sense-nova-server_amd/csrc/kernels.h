@@ -185,6 +185,8 @@ struct SpecArgs {
     int ring_n;
 };
 int launch_spec_next(const SpecArgs& a, hipStream_t s);
+// *d = h, in stream order
+int launch_put_step(const StepDev& h, StepDev* d, hipStream_t s);
 // host_out: pinned host memory (its device address) that also receives the picks
 int launch_pick(const float* logits, int V, int rows, float* scratch, Pick* out, hipStream_t s,
                 Pick* host_out = nullptr);

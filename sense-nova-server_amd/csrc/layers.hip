@@ -425,6 +425,20 @@ int launch_merge(float* x, const float* coef, const float* br, int h, int M, int
 
 size_t pick_scratch_floats(int V, int rows) { return (size_t)rows * ((V + kPickChunk - 1) / kPickChunk) * 3; }
 
+// A step record carried by the launch's own arguments: no copy and no wait for one (an upload and the
+// synchronisation that its pageable source needs took 11 us of a kernel-level call).
+__global__ __launch_bounds__(256) void put_step_kernel(StepDev h, StepDev* d) {
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(&h);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(d);
+    for (int i = threadIdx.x; i < (int)(sizeof(StepDev) / 4); i += 256) dst[i] = src[i];
+}
+static_assert(sizeof(StepDev) % 4 == 0 && sizeof(StepDev) < 4000, "a step record fits a launch's arguments");
+
+int launch_put_step(const StepDev& h, StepDev* d, hipStream_t s) {
+    hipLaunchKernelGGL(put_step_kernel, dim3(1), dim3(256), 0, s, h, d);
+    return last_error();
+}
+
 int launch_spec_next(const SpecArgs& a, hipStream_t s) {
     if (!a.vstep || !a.mstep || !a.picks || !a.draft || !a.rope_tab || a.rope_rows < 1 || !a.hid1 || !a.hlast ||
         a.h < 1 || !a.ring || a.ring_n < 1)
