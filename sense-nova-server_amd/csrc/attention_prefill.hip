@@ -294,6 +294,7 @@ static int part_keys(int M, int n_kv, int keys) {
 }
 
 size_t attention_prefill_part_floats(int ctx, int n_heads) {
+    if (ctx <= KPART_MIN) return 0;  // one part
     size_t most = 0;
     for (int m = QTILE; m <= SNL_PF_M; m += QTILE) {
         const int kp = part_keys(m, n_heads / G, ctx);

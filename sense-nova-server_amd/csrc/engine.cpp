@@ -689,10 +689,10 @@ int snl_engine::init() {
             (rc = dalloc(&pf_dk, P * std::max<size_t>(key_dim, 1))) || (rc = dalloc(&pf_dv, P * lin_value_dim + 1)) ||
             (rc = dalloc(&pf_gz, P * lin_value_dim + 1)) || (rc = dalloc(&pf_beta, P * nv)) ||
             (rc = dalloc(&pf_decay, P * nv)) || (rc = dalloc((uint8_t**)&pf_frags, frags_bytes(SNL_PF_M, kmax))) ||
-            (rc = dalloc(&pf_gpart, pf_gpart_n + 1)) || (rc = dalloc(&d_pstep, 1)))
+            (pf_gpart_n && (rc = dalloc(&pf_gpart, pf_gpart_n))) || (rc = dalloc(&d_pstep, 1)))
             return rc;
         pf_apart_n = attention_prefill_part_floats(ctx, c.n_heads);
-        if ((rc = dalloc(&pf_apart, pf_apart_n))) return rc;
+        if (pf_apart_n && (rc = dalloc(&pf_apart, pf_apart_n))) return rc;
         if (hipHostMalloc((void**)&h_pstep, sizeof(PrefillDev), hipHostMallocDefault) != hipSuccess)
             return fail(SNL_ENOMEM, "pinned host allocation failed");
     }

@@ -109,3 +109,28 @@ def test_worker_sampled(snl_mod, eng):
     z = w.run_sampled(prompt, 24, snl_mod.Sampling(temperature=0.0), seed=1)
     assert z["tokens"] == g["tokens"]
     w.close()
+
+
+@pytest.mark.parametrize("vocab", [40, 4095, 4097, 33001])
+def test_top_k_order(snl_mod, vocab):
+    """The device's k largest in the reference's order (value descending, index ascending), for k at
+    the edges of the wave lists and of the chunks, with most logits equal (a zeroed tail of the head)."""
+    import dataclasses
+
+    cfg = dataclasses.replace(snl_mod.tiny_config(), vocab=vocab)
+    e = snl_mod.Engine(cfg, seed=13, quant=0, ctx=64)
+    try:
+        for tied in (False, True):
+            if tied:
+                e.zero_rows(-1, snl_mod.engine.K_LM_HEAD, vocab - vocab // 2)
+            lg = _logits(e, cfg, vocab)[0]
+            order = np.lexsort((np.arange(vocab), -lg))
+            for k in (1, 2, 20, 63, 64, 65, 200):
+                k = min(k, vocab)
+                print(f"top-k vocab {vocab} k {k} tied {tied}", flush=True)
+                s = snl_mod.Sampler(e, snl_mod.Sampling(temperature=1.0, top_p=1.0, top_k=k), seed=1)
+                toks, _ = s.distribution(0)
+                assert toks.tolist() == order[:k].tolist()
+                s.close()
+    finally:
+        e.close()
