@@ -105,8 +105,7 @@ struct GemmArgs {
 size_t gemm_q_bytes(int quant, int N, int K);
 size_t gemm_s_floats(int N, int K);
 size_t frags_bytes(int M, int K);
-// slices of K, a rule on the matrix's shape alone; *slice_st: 64-element stages per slice
-int gemm_slices(int N, int K, int* slice_st);
+// partial sums that a launch of up to M rows may need
 size_t gemm_part_floats(int M, int N, int K);
 // reference layout (q [N, K] Q8 / [N, K/2] Q4, s [N, K/32]) -> panel order
 int launch_panel_pack(int quant, int N, int K, const void* q, const float* s, void* qp, float* sp, hipStream_t st);

@@ -30,8 +30,9 @@
 //
 // Each output element's arithmetic is fixed by its row and column, whatever M or the tile it falls
 // in, so a token's result does not depend on the chunk that carries it.  K is cut into slices by a
-// rule on (N, K) alone (gemm_slices); a slice's blocks are summed in order from zero and the slices
-// are added in order, whether one block runs them all or each is a block of its own.
+// rule on (N, K) alone (slices_of), the slices into groups; a slice's blocks are summed in order from
+// zero, a group's slices in order and the groups in order, whether one block runs them all or each
+// slice, or each group, is a block of its own.
 #include <algorithm>
 
 #include "common.h"
@@ -328,11 +329,18 @@ __device__ __forceinline__ void copy16_to_lds(const char* base, unsigned voff, u
                  : "memory", "m0");
 }
 
-// Slices: `slices` pieces of K of `slice_st` stages each (the last takes the rest).  SPLIT: a block
-// runs one slice and leaves its sums in a.part; else a block runs them all.
-template <int QT, int WT, int WR, int TTW, int RT, bool SPLIT>
+// What one block runs of its outputs' sums (struct Slices): all of K, or one slice or one group of
+// slices, whose sum it leaves in a.part.
+enum Split { WHOLE = 0, BY_SLICE = 1, BY_GROUP = 2 };
+struct Slices {
+    int n, st;         // slices, stages of each (the last takes the rest)
+    int groups, per;   // groups, slices of each
+    int run_st(int split) const { return split == BY_SLICE ? st : st * per; }
+    int runs(int split) const { return split == BY_SLICE ? n : groups; }
+};
+template <int QT, int WT, int WR, int TTW, int RT, int SPLIT>
 __global__ __launch_bounds__(WT * WR * 64) void mgemm_kernel(GemmArgs a, int r_first, int rpanels, int tpanels,
-                                                             int slices, int slice_st) {
+                                                             Slices sl) {
     using G = GemmStage<QT, WT, WR, TTW, RT>;
     extern __shared__ __align__(16) uint4 lds[];  // D stage buffers of G::U4
     // the wave index in a scalar register: the copies' addresses then form in scalar code
@@ -340,17 +348,19 @@ __global__ __launch_bounds__(WT * WR * 64) void mgemm_kernel(GemmArgs a, int r_f
     const int wt = wave / G::WR, wr = wave % G::WR;
     // XCD-aware numbering: block b runs on XCD b % 8; give each XCD whole row panels (SPLIT: whole
     // slices of row panels), whose weights its L2 then serves to every token panel
-    const int units = SPLIT ? rpanels * slices : rpanels;
+    const int runs = SPLIT == BY_SLICE ? sl.n : SPLIT == BY_GROUP ? sl.groups : 1;
+    const int units = rpanels * runs;
     const int bid = blockIdx.x;
     const int xcd = bid & 7, idx = bid >> 3;
     const int per_xcd = (units + 7) / 8;
     const int unit = xcd * per_xcd + idx / tpanels;
     const int tp = idx % tpanels;
     if (unit >= units) return;
-    const int rp = SPLIT ? unit / slices : unit, z = SPLIT ? unit % slices : 0;
+    const int rp = SPLIT ? unit / runs : unit, z = SPLIT ? unit % runs : 0;
     const int nb = a.K / 32, nst_all = a.K / 64;
-    const int st0 = SPLIT ? z * slice_st : 0;
-    const int nst = SPLIT ? min(slice_st, nst_all - st0) : nst_all;
+    const int run_st = SPLIT == BY_SLICE ? sl.st : sl.st * sl.per;
+    const int st0 = SPLIT ? z * run_st : 0;
+    const int nst = SPLIT ? min(run_st, nst_all - st0) : nst_all;
     const int j = lane & 31, g = lane >> 5;
     const int R0 = r_first + rp * G::BR, T0 = tp * G::TT;
 
@@ -401,11 +411,12 @@ __global__ __launch_bounds__(WT * WR * 64) void mgemm_kernel(GemmArgs a, int r_f
         else wait_stages<G::WC, G::D - 2 * G::PS, G::PS>(n);
     };
 
-    f32x16_t acc[RT][TTW], tot[RT][TTW];
+    // the running sums of the slice, of the group and of all groups
+    f32x16_t acc[RT][TTW], grp[RT][TTW], tot[RT][TTW];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int t = 0; t < TTW; ++t) acc[r][t] = tot[r][t] = f32x16_t{};
+        for (int t = 0; t < TTW; ++t) acc[r][t] = grp[r][t] = tot[r][t] = f32x16_t{};
 
     half8_t x[2][TTW][4];  // [block of the stage][token tile][2 * half + (0 hi, 1 lo)]
     uint4 wv[2][RT][G::PB];  // [stage % 2]; Q8: the two blocks' bytes; Q4: both blocks' words
@@ -493,7 +504,7 @@ __global__ __launch_bounds__(WT * WR * 64) void mgemm_kernel(GemmArgs a, int r_f
         __builtin_amdgcn_sched_barrier(0);
     };
     enter(0);
-    int buf = 0, left = SPLIT ? 0 : slice_st;
+    int buf = 0, left = sl.st, left_g = sl.per;
     read_weights(0, lds);
     read_block(0, lds);
     wh[0][0] = dequant(0, 0, 0, 0);
@@ -521,9 +532,9 @@ __global__ __launch_bounds__(WT * WR * 64) void mgemm_kernel(GemmArgs a, int r_f
             __builtin_amdgcn_sched_barrier(0);
         }
         multiply(p, 1);
-        if constexpr (!SPLIT && RT * TTW <= 2) {
+        if constexpr (SPLIT != BY_SLICE && RT * TTW <= 2) {
             if (--left == 0) {
-                left = slice_st;
+                left = sl.st;
                 scale(1, RT - 1, TTW - 1);
                 dsc = 0.0f;
                 d[1] = f32x16_t{};
@@ -531,9 +542,19 @@ __global__ __launch_bounds__(WT * WR * 64) void mgemm_kernel(GemmArgs a, int r_f
                 for (int r = 0; r < RT; ++r)
 #pragma unroll
                     for (int t = 0; t < TTW; ++t) {
-                        tot[r][t] = tot[r][t] + acc[r][t];
+                        grp[r][t] = grp[r][t] + acc[r][t];
                         acc[r][t] = f32x16_t{};
                     }
+                if (SPLIT == WHOLE && --left_g == 0) {
+                    left_g = sl.per;
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)
+#pragma unroll
+                        for (int t = 0; t < TTW; ++t) {
+                            tot[r][t] = tot[r][t] + grp[r][t];
+                            grp[r][t] = f32x16_t{};
+                        }
+                }
             }
         }
     };
@@ -554,26 +575,32 @@ __global__ __launch_bounds__(WT * WR * 64) void mgemm_kernel(GemmArgs a, int r_f
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
                 const int n = 32 * (R0 + wr * RT + r) + j;
-                if (n < a.N) yr[n] = SPLIT ? acc[r][t][i] : (tot[r][t][i] + acc[r][t][i]) * xs;
+                if (n >= a.N) continue;
+                const float sum = SPLIT == BY_SLICE ? acc[r][t][i] : grp[r][t][i] + acc[r][t][i];
+                yr[n] = SPLIT ? sum : (tot[r][t][i] + sum) * xs;
             }
         }
     }
 }
 
-// y[m, n] = (sum of the slices' partials in slice order) * xs[m]
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, int slices) {
+// y[m, n] = xs[m] * the sum over groups, in order, of each group's n partials summed in order
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, int n_part, int per) {
     const int m = blockIdx.y, n = blockIdx.x * 256 + threadIdx.x;
     if (n >= a.N) return;
     const float* p = a.part + (size_t)m * a.N + n;
     const size_t step = (size_t)a.M * a.N;
     float t = 0.0f;
-    for (int z = 0; z < slices; ++z) t = t + p[z * step];
+    for (int z = 0; z < n_part;) {
+        float g = 0.0f;
+        for (int e = min(n_part, z + per); z < e; ++z) g = g + p[z * step];
+        t = t + g;
+    }
     a.y[(size_t)m * a.y_stride + a.n_off + n] = t * a.xs[m];
 }
 
 // Row tiles [r_first, r_first + r_count) of the matrix.
-template <int QT, int WT, int WR, int TTW, int RT, bool SPLIT>
-int gemm_launch(const GemmArgs& a, int r_first, int r_count, int slices, int slice_st, hipStream_t s) {
+template <int QT, int WT, int WR, int TTW, int RT, int SPLIT>
+int gemm_launch(const GemmArgs& a, int r_first, int r_count, const Slices& sl, hipStream_t s) {
     using G = GemmStage<QT, WT, WR, TTW, RT>;
     const auto kernel = &mgemm_kernel<QT, WT, WR, TTW, RT, SPLIT>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -581,10 +608,12 @@ int gemm_launch(const GemmArgs& a, int r_first, int r_count, int slices, int sli
     if (attr != hipSuccess) return -2;
     const int mtiles = (a.M + 31) / 32;
     const int rpanels = (r_count + G::BR - 1) / G::BR, tpanels = (mtiles + G::TT - 1) / G::TT;
-    const int units = SPLIT ? rpanels * slices : rpanels;
+    const int units = SPLIT ? rpanels * sl.runs(SPLIT) : rpanels;
     const int blocks = 8 * ((units + 7) / 8) * tpanels;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(G::NW * 64), G::BYTES, s, a, r_first, rpanels, tpanels, slices, slice_st);
-    if (SPLIT) hipLaunchKernelGGL(gemm_reduce_kernel, dim3((a.N + 255) / 256, a.M), dim3(256), 0, s, a, slices);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(G::NW * 64), G::BYTES, s, a, r_first, rpanels, tpanels, sl);
+    if (SPLIT)
+        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((a.N + 255) / 256, a.M), dim3(256), 0, s, a, sl.runs(SPLIT),
+                           SPLIT == BY_SLICE ? sl.per : 1);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -594,20 +623,38 @@ int xcd_rounds(int panels, int tpanels) { return ((panels + 7) / 8 * tpanels + 3
 // Microseconds of one round of blocks at K = 4096 (Q8, all CUs busy): 128 x 256, 128 x 128 and
 // 64 x 128 blocks.  What a launch costs is its rounds times this; only the proportions matter.
 constexpr int kRoundWide = 127, kRoundMid = 67, kRoundNarrow = 44;
+// and what two groups of slices and the addition of their sums cost beside one of all K (4096 x 4096, 512
+// rows: 50 us one block, 51 by group; 4096 x 12288: 145 and 126)
+constexpr int kReduce = 14;
+
+// The slices of K, a rule on the matrix's shape alone.  Four or more form two groups.
+Slices slices_of(int N, int K) {
+    const int p = (N + 127) / 128, q = K / 128;
+    const int s = p >= 46 ? 1 : std::max(1, std::min({8, 256 / p, K / kSliceMin}));
+    const int len = (q + s - 1) / s;  // slices in units of 128 elements
+    const int n = (q + len - 1) / len, per = n >= 4 ? (n + 1) / 2 : n;
+    return Slices{n, 2 * len, (n + per - 1) / per, per};
+}
 
 template <int QT>
 int gemm_dispatch(const GemmArgs& a, hipStream_t s) {
     const int rt = (a.N + 31) / 32, mtiles = (a.M + 31) / 32;
-    int slice_st;
-    const int slices = gemm_slices(a.N, a.K, &slice_st);
-    if (slices > 1) {
+    const Slices sl = slices_of(a.N, a.K);
+    if (sl.n > 1) {
         if (a.part && (rt + 3) / 4 * ((mtiles + 1) / 2) <= kSplitPanels) {
-            if (mtiles <= 1) return gemm_launch<QT, 1, 4, 1, 1, true>(a, 0, rt, slices, slice_st, s);
-            return gemm_launch<QT, 2, 4, 1, 1, true>(a, 0, rt, slices, slice_st, s);
+            if (mtiles <= 1) return gemm_launch<QT, 1, 4, 1, 1, BY_SLICE>(a, 0, rt, sl, s);
+            return gemm_launch<QT, 2, 4, 1, 1, BY_SLICE>(a, 0, rt, sl, s);
         }
-        return gemm_launch<QT, 2, 4, 1, 1, false>(a, 0, rt, slices, slice_st, s);
+        // Many rows: 64 x 128 blocks over all of K, or 128 x 128 ones over a group of slices each, which
+        // read the LDS half as often per product, and kReduce to add the groups' sums.
+        const int pn = (rt + 3) / 4;
+        const int whole = xcd_rounds(pn, (mtiles + 1) / 2) * kRoundNarrow * 2;
+        const int by_group = xcd_rounds(pn * sl.groups, (mtiles + 3) / 4) * kRoundMid * 2 / sl.groups;
+        if (a.part && sl.groups > 1 && by_group * (a.K / 128) + 2 * kReduce * 32 < whole * (a.K / 128))
+            return gemm_launch<QT, 2, 4, 2, 1, BY_GROUP>(a, 0, rt, sl, s);
+        return gemm_launch<QT, 2, 4, 1, 1, WHOLE>(a, 0, rt, sl, s);
     }
-    if (mtiles <= 1) return gemm_launch<QT, 1, 4, 1, 1, false>(a, 0, rt, 1, slice_st, s);
+    if (mtiles <= 1) return gemm_launch<QT, 1, 4, 1, 1, WHOLE>(a, 0, rt, sl, s);
     // The block size by the rounds each needs: the last one costs as much as a full one.  Whole rounds
     // of 128 x 256 blocks may leave their remainder to 128 x 128 ones.
     const int tw = (mtiles + 3) / 4, tn = (mtiles + 1) / 2, pw = (rt + 7) / 8, pn = (rt + 3) / 4;
@@ -616,11 +663,11 @@ int gemm_dispatch(const GemmArgs& a, hipStream_t s) {
     const int head = (rw - 1) * 32 / tw * 8;  // panels of the whole rounds
     const int mixed = rw > 1 && head > 0 && head < pw
                           ? xcd_rounds(head, tw) * kRoundWide + xcd_rounds((rt - 8 * head + 3) / 4, tw) * kRoundMid : wide;
-    if (narrow <= mid && narrow <= wide && narrow <= mixed) return gemm_launch<QT, 2, 4, 1, 1, false>(a, 0, rt, 1, slice_st, s);
-    if (mid < wide && mid <= mixed) return gemm_launch<QT, 2, 4, 2, 1, false>(a, 0, rt, 1, slice_st, s);
-    if (wide <= mixed) return gemm_launch<QT, 2, 4, 2, 2, false>(a, 0, rt, 1, slice_st, s);
-    const int rc = gemm_launch<QT, 2, 4, 2, 2, false>(a, 0, 8 * head, 1, slice_st, s);
-    return rc ? rc : gemm_launch<QT, 2, 4, 2, 1, false>(a, 8 * head, rt - 8 * head, 1, slice_st, s);
+    if (narrow <= mid && narrow <= wide && narrow <= mixed) return gemm_launch<QT, 2, 4, 1, 1, WHOLE>(a, 0, rt, sl, s);
+    if (mid < wide && mid <= mixed) return gemm_launch<QT, 2, 4, 2, 1, WHOLE>(a, 0, rt, sl, s);
+    if (wide <= mixed) return gemm_launch<QT, 2, 4, 2, 2, WHOLE>(a, 0, rt, sl, s);
+    const int rc = gemm_launch<QT, 2, 4, 2, 2, WHOLE>(a, 0, 8 * head, sl, s);
+    return rc ? rc : gemm_launch<QT, 2, 4, 2, 1, WHOLE>(a, 8 * head, rt - 8 * head, sl, s);
 }
 
 }  // namespace
@@ -632,18 +679,11 @@ size_t gemm_q_bytes(int quant, int N, int K) { return panel_tiles(N) * (quant ==
 
 size_t gemm_s_floats(int N, int K) { return panel_tiles(N) * 32 * (K / 32); }
 
-int gemm_slices(int N, int K, int* slice_st) {
-    const int p = (N + 127) / 128, q = K / 128;
-    int s = p >= 46 ? 1 : std::max(1, std::min({8, 256 / p, K / kSliceMin}));
-    const int len = (q + s - 1) / s;  // slices in units of 128 elements
-    *slice_st = 2 * len;
-    return (q + len - 1) / len;
-}
-
 size_t gemm_part_floats(int M, int N, int K) {
-    int st;
-    const int s = gemm_slices(N, K, &st), p = (N + 127) / 128;
-    return s > 1 ? (size_t)s * std::min(M, kSplitPanels / p * 64) * N : 0;
+    const Slices sl = slices_of(N, K);
+    if (sl.n == 1) return 0;
+    const int p = (N + 127) / 128;
+    return std::max((size_t)sl.n * std::min(M, kSplitPanels / p * 64), (size_t)(sl.groups > 1 ? sl.groups * M : 0)) * N;
 }
 
 int launch_panel_pack(int quant, int N, int K, const void* q, const float* s, void* qp, float* sp, hipStream_t st) {

@@ -137,6 +137,8 @@ def test_gemm_rows_independent_of_m(torch_cuda, K, oracle, quant):
     (8200, 384, (129, 128, 65, 64)),     # 128 x 128 and 64 x 128 blocks
     (5760, 1152, (193, 129, 128, 5)),    # two slices, the most panels that have any
     (4096, 1664, (512, 193, 192, 31)),   # slices of 5, 5 and 3: run by one block, and split over blocks
+    (4096, 2176, (512, 257, 160, 7)),    # four slices, the last short, in two groups: one block, by slice
+    (2050, 4096, (511, 300, 65)),        # eight slices in two groups, ragged panels: by group, by slice
     (13, 512, (65, 2)), (256, 768, (300,)), (136, 4096, (512, 40, 3))])
 def test_gemm_block_shapes(torch_cuda, K, oracle, quant, n, k, rows):
     """Every block shape and slice form of the prefill GEMM, at the edges of their ranges: against
