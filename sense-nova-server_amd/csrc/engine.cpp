@@ -2066,19 +2066,21 @@ int snl_gemv(int quant, const void* wq, const float* ws, const float* x, float* 
     g.K = K;
     g.epi = GEMV_STORE;
     // A Q8 matrix is read where it lies (gemv.hip): packing it into the tile order of the engine's kernel
-    // for one product cost more than the product (2 rows, us a call packed / direct: 12352 x 4096 57 /
-    // 33, 24576 x 4096 87 / 38, 1544 x 256 23 / 18).  Q4 keeps the engine's kernel, and with it the
-    // engine's rounding (its -8 x block sum correction, 2e-6 of a result against 1e-7); so do quants that
-    // 16-byte loads cannot read.  Those are packed into a staging buffer, held under the lock until the
-    // call has finished on the stream.  Shapes of the engine's kernel return when their work is done, the
-    // others when it is queued.
+    // for one product cost more than the product (2 rows, us a call packed / direct: 12352 x 4096 56 /
+    // 30, 24576 x 4096 87 / 38, 4096 x 12288 56 / 38), with less rounding (1.25e-7 -> 9.6e-8 of the
+    // result, 1.24e-7 -> 1.09e-7 at K = 12288).  The engine's kernel keeps rows shorter than 1024, where a
+    // call is mostly its launch and wait and exact block sums round less (K = 256: 7.8e-8 against 8.2e-8),
+    // and Q4, with the engine's rounding (its -8 x block sum correction, 2e-6 of a result against 1e-7);
+    // also quants that 16-byte loads cannot read.  These are packed into a staging buffer, held under the
+    // lock until the call has finished on the stream.  Shapes of the engine's kernel return when their
+    // work is done, the others when it is queued.
     static uint8_t* pq = nullptr;
     static float* ps = nullptr;
     static size_t cap_q = 0, cap_s = 0;
     std::lock_guard<std::mutex> lk(g_kstep_mu);
     PackGeom pg;
     const bool waits = pack_geom(quant, N, K, 0, &pg) && M >= 1 && M <= SNL_MAX_M && mgemv_fits(M, K);
-    if (waits && (quant != 0 || (uintptr_t)wq % 16)) {
+    if (waits && (quant != 0 || K < 1024 || (uintptr_t)wq % 16)) {
         if (pg.q_bytes > cap_q || pg.s_floats > cap_s) {
             if (hipStreamSynchronize(st) != hipSuccess) return SNL_EDEVICE;
             hipFree(pq);

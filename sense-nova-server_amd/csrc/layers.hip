@@ -1,4 +1,4 @@
-// Norms, mHC routing, residual merges, SwiGLU, embedding gather and the greedy pick.
+// Norms, mHC routing, residual merges, embedding gather and the greedy pick.
 // Semantics follow src/shaders/layers.wgsl, src/engine.rs:777-790 and src/sampler.rs:169-177.
 #include <float.h>
 

@@ -59,7 +59,8 @@ def test_gemv_matches_oracle(torch_cuda, K, oracle, quant, n, k, m):
     assert np.all(np.abs(got - exact) <= 1e-5 * scale + 1e-7)
 
 
-@pytest.mark.parametrize("quant,n,k", [(0, 12352, 4096), (0, 13, 128), (0, 16411, 1152), (0, 65537, 256), (0, 21, 1056),
+@pytest.mark.parametrize("quant,n,k", [(0, 12352, 4096), (0, 13, 1024), (0, 16411, 1152), (0, 65537, 1024), (0, 40, 896),
+                                       (0, 21, 1056),
                                        (1, 21, 1056), (1, 40, 32)])
 def test_gemv_row_major(torch_cuda, K, oracle, quant, n, k):
     """Weights read where they lie, at the edges of the row groups and K chunks, and a Q8 matrix that
