@@ -25,6 +25,8 @@
 // matrix-core kernel (mgemv.hip) is faster on weights laid out once, but packing a matrix into tile
 // order for a single product moves it three times.
 // It computes the plain product y = W x.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -58,18 +60,6 @@ __device__ __forceinline__ void load_frag(const GemvArgs& a, int row, int k, uin
     } else {
         w[0] = w[1] = w[2] = w[3] = QT == 0 ? 0u : 0x88888888u;
         sc = 0.0f;
-    }
-}
-
-// the lane's 16 quants as exact f32 (Q8: signed bytes; Q4: nibble - 8, as the signed 4 bits of nibble ^ 8)
-template <int QT>
-__device__ __forceinline__ void quants16(const uint32_t (&w)[4], float (&q)[16]) {
-    if constexpr (QT == 0) {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) q[j] = (float)(int8_t)(w[j / 4] >> (8 * (j % 4)));
-    } else {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) q[j] = (float)((int)((w[j / 8] ^ 0x88888888u) << (28 - 4 * (j % 8))) >> 28);
     }
 }
 
@@ -138,18 +128,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a, int G) {
                 float q[16];
                 quants16<QT>(wc[r], q);
 #pragma unroll
-                for (int m = 0; m < M; ++m) {
-                    // four sums of four, added in pairs: shorter chains round less than one of 16 (9.6e-8 of
-                    // a result at K = 4096 against 1.07e-7) and wait less (33 -> 30 us a call at 12352 x 4096)
-                    float p[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        p[e] = q[e] * xv[m][e];
-#pragma unroll
-                        for (int f = 4; f < 16; f += 4) p[e] = fmaf(q[e + f], xv[m][e + f], p[e]);
-                    }
-                    acc[r][m] = fmaf(scc[r], (p[0] + p[1]) + (p[2] + p[3]), acc[r][m]);
-                }
+                for (int m = 0; m < M; ++m) acc[r][m] = fmaf(scc[r], dot16(q, xv[m]), acc[r][m]);
             }
         }
         if (c == nchunks - 1) {
@@ -211,6 +190,9 @@ int groups_for(int N) {
     return 1;
 }
 
+// floats of a token row staged in LDS, whole chunks
+size_t row_floats(int K) { return (size_t)(K + kChunk - 1) / kChunk * kChunk; }
+
 }  // namespace
 
 int gemv_init() {
@@ -235,8 +217,9 @@ int launch_gemv(const GemvArgs& a, int quant, int M, hipStream_t s) {
     }
     // row-major weights: the plain product only
     if (a.epi != GEMV_STORE || a.pro != GEMV_PLAIN) return -1;
-    const int K4p = (a.K + kChunk - 1) / kChunk * (kChunk / 4);
-    if ((size_t)M * K4p * 4 > (size_t)kLdsFloats) {
+    // Longer rows go to gemv_ksplit.hip, one row where two do, so that it gives a two-row call's bits (and
+    // faster: 17792 x 4096, one row 39 us here, 33 there)
+    if (std::max(M, 2) * row_floats(a.K) > (size_t)kLdsFloats) {
         if (a.row_base) return -1;
         return launch_gemv_ksplit(a, quant, M, s);
     }
@@ -244,7 +227,7 @@ int launch_gemv(const GemvArgs& a, int quant, int M, hipStream_t s) {
     if (!f) return -1;
     const int G = groups_for(a.N);
     dim3 grid((a.N + 16 * G - 1) / (16 * G));
-    const size_t lds = (size_t)M * K4p * 16;
+    const size_t lds = M * row_floats(a.K) * 4;
     hipLaunchKernelGGL(f, grid, dim3(kThreads), lds, s, a, G);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }

@@ -1,5 +1,5 @@
 // K-split skinny GEMV (fallback for shapes whose token rows do not fit the LDS of the
-// streaming kernel in gemv.hip: M*K > 32768 floats), gfx950.
+// streaming kernel in gemv.hip: M*K > 32768 floats; one row goes where two do), gfx950.
 //
 // y[m, n] = sum_b s[n, b] * sum_{i<32} q[n, 32b + i] * x[m, 32b + i]
 //
@@ -15,10 +15,9 @@
 // them to all 16 weight rows: the weights are read once for every token row (the M=2
 // verify pass costs the weight bytes of one pass).
 //
-// Dequantisation in registers.  Q8: the word is xor-ed with 0x80808080, which turns
-// each int8 q into the unsigned byte q+128; v_cvt_f32_ubyte{0..3} converts one byte per
-// instruction and the bias is removed once per half-block, sum (q+128) x - 128 sum x.
-// Q4: the nibbles n are masked into bytes and converted the same way, minus 8 sum x.
+// Dequantisation in registers: each quant is converted once, exactly, and multiplied with every token
+// row's element, as in gemv.hip.  (Bytes as q + 128 with the bias taken off as 128 sum x cancel: two rows
+// at K = 16512 were 3.1e-7 of the result off, 1.08e-7 so, in the same time, 37 us at N = 4096.)
 //
 // Reduction.  Each lane holds 16 row partials per token row; a transposed butterfly
 // (xor 32, 16, 8, 4 exchange half of the values, then xor 2, 1 add) leaves lane 4r with
@@ -43,30 +42,6 @@ constexpr int kChunk = 1024;
 
 __device__ __forceinline__ int row_of(int blk, int r) { return blk * kRows + r; }
 
-// sum over the lane's 16 products of (byte value) * x, for one token row
-template <int QT>
-__device__ __forceinline__ void dot16(const uint32_t (&w)[4], const float (&x)[16], float& p) {
-    if constexpr (QT == 0) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t u = w[j] ^ 0x80808080u;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) p = fmaf((float)((u >> (8 * b)) & 0xFFu), x[4 * j + b], p);
-        }
-    } else {
-        // two words = 16 nibbles = elements 0..15 of the lane's half block
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            uint32_t lo = w[j] & 0x0F0F0F0Fu, hi = (w[j] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                p = fmaf((float)((lo >> (8 * b)) & 0xFFu), x[8 * j + 2 * b], p);
-                p = fmaf((float)((hi >> (8 * b)) & 0xFFu), x[8 * j + 2 * b + 1], p);
-            }
-        }
-    }
-}
-
 template <int QT, int M>
 __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -83,7 +58,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a) {
     for (int c = wave; c < nchunks; c += 4) {
         const int k = c * kChunk + lane * 16;
         if (k < K) {
-            float xs[M][16], sx[M];
+            float xs[M][16];
 #pragma unroll
             for (int m = 0; m < M; ++m) {
                 const float4* xp = reinterpret_cast<const float4*>(a.x + (size_t)m * a.x_stride + k);
@@ -95,12 +70,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a) {
                     xs[m][4 * v + 2] = t.z;
                     xs[m][4 * v + 3] = t.w;
                 }
-                float s = xs[m][0];
-#pragma unroll
-                for (int i = 1; i < 16; ++i) s = s + xs[m][i];
-                sx[m] = s;
             }
-            const float bias = QT == 0 ? 128.0f : 8.0f;
 #pragma unroll
             for (int r0 = 0; r0 < kRows; r0 += 8) {
                 uint32_t wv[8][4];
@@ -121,18 +91,18 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(GemvArgs a) {
                         }
                         sc[r] = a.ws[(size_t)row * nb + (k >> 5)];
                     } else {
-                        wv[r][0] = wv[r][1] = wv[r][2] = wv[r][3] = QT == 0 ? 0x80808080u : 0x88888888u;
+                        wv[r][0] = wv[r][1] = wv[r][2] = wv[r][3] = QT == 0 ? 0u : 0x88888888u;
                         sc[r] = 0.0f;
                     }
                 }
 #pragma unroll
-                for (int r = 0; r < 8; ++r)
+                for (int r = 0; r < 8; ++r) {
+                    float q[16];
+                    quants16<QT>(wv[r], q);
 #pragma unroll
-                    for (int m = 0; m < M; ++m) {
-                        float p = 0.0f;
-                        dot16<QT>(wv[r], xs[m], p);
-                        acc[r0 + r][m] = fmaf(sc[r], fmaf(-bias, sx[m], p), acc[r0 + r][m]);
-                    }
+                    for (int m = 0; m < M; ++m)
+                        acc[r0 + r][m] = fmaf(sc[r], dot16(q, xs[m]), acc[r0 + r][m]);
+                }
             }
         }
     }

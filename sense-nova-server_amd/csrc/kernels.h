@@ -58,9 +58,9 @@ struct GemvArgs {
 int mgemv_blocks(int quant, int N, int K, int inter);
 // The matrix-core path for tile-order weights, the vector-ALU kernels of gemv.hip / gemv_ksplit.hip for
 // the reference's row-major layout (kernel-level calls only: snl_gemv on Q8 at K >= 1024, and at shapes the
-// matrix-core kernel does not serve, K % 128 != 0 or M = 3, 4 where two token pairs overflow LDS).
+// matrix-core kernel does not serve, K % 128 != 0 or M = 3, 4 at K > 4096).
 int launch_gemv(const GemvArgs& a, int quant, int M, hipStream_t s);
-// vector-ALU fallback, K split over blocks (kernel-level calls only)
+// token rows too long for the LDS of gemv.hip, K split over waves (kernel-level calls only)
 int launch_gemv_ksplit(const GemvArgs& a, int quant, int M, hipStream_t s);
 // Matrix-core path (mgemv.hip) over tile-order weights: 0 launched, 1 not served (M too large for
 // LDS at this K), < 0 error.

@@ -90,6 +90,28 @@ def test_gemv_row_major(torch_cuda, K, oracle, quant, n, k):
         assert np.array_equal(y1.cpu().numpy()[0], got[1, :n])
 
 
+@pytest.mark.parametrize("n,k", [(40, 16384), (40, 16512), (21, 16896), (13, 17792)])
+def test_gemv_long_rows(torch_cuda, K, oracle, n, k):
+    """Two Q8 rows at the lengths where they no longer fit the LDS of gemv.hip: bitwise the one-row calls,
+    and within 2e-6 of the sum of |terms| (the float64 product; test_gemv_row_major's bound)."""
+    torch = torch_cuda
+    print(f"gemv long rows n={n} k={k}", flush=True)
+    q, s, x = _gemv_case(oracle, 0, n, k, 2, seed=n + k)
+    deq = oracle.dequant(q, s, 0, k).astype(np.float64)
+    exact, scale = x.astype(np.float64) @ deq.T, np.abs(x.astype(np.float64)) @ np.abs(deq).T
+    dq, ds, dx = _dev(torch, q), _dev(torch, s), _dev(torch, x)
+    y = torch.zeros((2, n), dtype=torch.float32, device="cuda")
+    K.gemv(0, dq, ds, dx, y, 2, n, k, k, n)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.all(np.abs(got - exact) <= 2e-6 * scale)
+    for m in range(2):
+        y1 = torch.zeros((1, n), dtype=torch.float32, device="cuda")
+        K.gemv(0, dq, ds, dx[m:], y1, 1, n, k, k, n)
+        torch.cuda.synchronize()
+        assert np.array_equal(y1.cpu().numpy()[0], got[m])
+
+
 @pytest.mark.parametrize("quant", [0, 1])
 @pytest.mark.parametrize("n,k,m", [(96, 1024, 3), (4096, 4096, 512), (1544, 256, 37), (12352, 4096, 130),
                                    (4096, 12288, 64), (24576, 4096, 17)])
