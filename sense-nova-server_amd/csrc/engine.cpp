@@ -2080,6 +2080,7 @@ int snl_gemv(int quant, const void* wq, const float* ws, const float* x, float* 
     std::lock_guard<std::mutex> lk(g_kstep_mu);
     PackGeom pg;
     const bool waits = pack_geom(quant, N, K, 0, &pg) && M >= 1 && M <= SNL_MAX_M && mgemv_fits(M, K);
+    if (waits && (uintptr_t)x % 16) return SNL_EARG;  // either kernel reads x in 16-byte pieces
     if (waits && (quant != 0 || K < 1024 || (uintptr_t)wq % 16)) {
         if (pg.q_bytes > cap_q || pg.s_floats > cap_s) {
             if (hipStreamSynchronize(st) != hipSuccess) return SNL_EDEVICE;

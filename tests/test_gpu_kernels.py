@@ -112,6 +112,30 @@ def test_gemv_long_rows(torch_cuda, K, oracle, n, k):
         assert np.array_equal(y1.cpu().numpy()[0], got[m])
 
 
+@pytest.mark.parametrize("quant,k", [(0, 256), (0, 1024), (0, 16512), (1, 1024)])
+def test_gemv_refuses_unaligned_x(torch_cuda, K, quant, k):
+    """Token rows off a 16-byte boundary are refused at every shape of the engine's kernel (K % 128 == 0),
+    whichever kernel takes the call, before anything is launched."""
+    import snl
+
+    torch = torch_cuda
+    n = 32
+    print(f"gemv unaligned x quant={quant} k={k}", flush=True)
+    q = torch.zeros((n, k if quant == 0 else k // 2), dtype=torch.uint8, device="cuda")
+    s = torch.zeros((n, k // 32), device="cuda")
+    x = torch.zeros(2 * k + 4, device="cuda")
+    y = torch.full((2, n), -7.0, device="cuda")
+    for off in (1, 2, 3):
+        with pytest.raises(snl.SnlError) as ei:
+            K.gemv(quant, q, s, x[off:], y, 2, n, k, k, n)
+        assert ei.value.code == snl.engine.SNL_EARG
+    torch.cuda.synchronize()
+    assert bool((y == -7.0).all())
+    K.gemv(quant, q, s, x[4:], y, 2, n, k, k, n)
+    torch.cuda.synchronize()
+    assert bool((y == 0).all())
+
+
 @pytest.mark.parametrize("quant", [0, 1])
 @pytest.mark.parametrize("n,k,m", [(96, 1024, 3), (4096, 4096, 512), (1544, 256, 37), (12352, 4096, 130),
                                    (4096, 12288, 64), (24576, 4096, 17)])
