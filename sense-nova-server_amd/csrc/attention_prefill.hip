@@ -294,7 +294,7 @@ static int part_keys(int M, int n_kv, int keys) {
 }
 
 size_t attention_prefill_part_floats(int ctx, int n_heads) {
-    if (ctx <= KPART_MIN) return 0;  // one part
+    if (ctx <= KPART_MIN || n_heads < G) return 0;  // one part, or a model without attention
     size_t most = 0;
     for (int m = QTILE; m <= SNL_PF_M; m += QTILE) {
         const int kp = part_keys(m, n_heads / G, ctx);
@@ -307,7 +307,7 @@ size_t attention_prefill_part_floats(int ctx, int n_heads) {
 
 int launch_attention_prefill(const AttnArgs& a, const PrefillDev* pstep, int M, int keys, float* part,
                              size_t part_floats, hipStream_t s) {
-    if (M < 1 || M > SNL_PF_M || a.n_heads != G * a.n_kv || a.rot_dim > HD || a.rot_dim % 2 || !pstep) return -1;
+    if (M < 1 || M > SNL_PF_M || a.n_kv < 1 || a.n_heads != G * a.n_kv || a.rot_dim > HD || a.rot_dim % 2 || !pstep) return -1;
     const int kpart = part_keys(M, a.n_kv, keys);
     const int parts = (keys + kpart - 1) / kpart;  // parts of the pass's longest key range
     if (parts > 1 && (!part || (size_t)M * a.n_heads * parts * (HD + 2) > part_floats)) return -1;

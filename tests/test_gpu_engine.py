@@ -445,6 +445,26 @@ def test_long_prefill_matches_decode_feed(snl_mod):
         e.close()
 
 
+def test_model_without_attention_heads(snl_mod, oracle):
+    """DeltaNet layers alone, no attention heads and no MTP head: built, and its logits are the oracle's."""
+    import dataclasses
+
+    cfg = dataclasses.replace(snl_mod.tiny_config(), full_attention=[False] * 8, n_heads=0, n_kv_heads=0, has_mtp=False)
+    print("model without attention heads", flush=True)
+    e = snl_mod.Engine(cfg, seed=5, quant=0, ctx=512)
+    o = oracle.Engine(cfg, seed=5, quant=0, ctx=512, max_m=e.prefill_chunk)
+    try:
+        prompt = _prompt(37, cfg.vocab, seed=8)
+        pos = [[i] * 3 for i in range(37)]
+        lg, _ = e.forward(prompt, pos, logit_rows=1)
+        ref = o.forward(prompt, pos, logit_rows=1)
+        ref = ref[0] if isinstance(ref, tuple) else ref
+        assert np.abs(lg - ref).max() / np.abs(ref).max() < 1e-3
+    finally:
+        e.close()
+        o.close()
+
+
 @pytest.mark.parametrize("prefix,rows", [(125, 3), (126, 3), (250, 17), (251, 16), (623, 33), (100, 512)])
 def test_prefill_attention_key_parts(snl_mod, prefix, rows):
     """A prefill pass over cached keys splits them into parts of at least 128 keys; at the parts'
