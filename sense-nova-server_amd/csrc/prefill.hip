@@ -122,6 +122,24 @@ __device__ __forceinline__ f32x4_t mfma16(const float4& xv, const float4& yv, f3
 }
 __device__ __forceinline__ float4 as_float4(f32x4_t v) { return make_float4(v[0], v[1], v[2], v[3]); }
 
+// acc + L X of a lower triangular L (lv: columns 4g .. 4g + 3 of row l % 16) and X in accumulator layout
+// (row 4g + i).  The product adds 0 x the rows past a row's own, which is NaN where such a row is not
+// finite: then each row is formed with those rows taken as 0, so a token never sees a later one.
+__device__ __forceinline__ f32x4_t lower16(const float4& lv, f32x4_t x, f32x4_t acc, int g) {
+    const float mag = (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3]));
+    if (!__any(!(mag < INFINITY))) return mfma16(lv, as_float4(x), acc);
+    f32x4_t out = {};
+    for (int b = 0; b < 16; ++b) {
+        f32x4_t xb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xb[i] = 4 * g + i <= b ? x[i] : 0.0f;
+        const f32x4_t y = mfma16(lv, as_float4(xb), acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = 4 * g + i == b ? y[i] : out[i];
+    }
+    return out;
+}
+
 __global__ __launch_bounds__(64) void dn_block_kernel(DnPrefillArgs a, int M) {
     __shared__ float kk[kBlk][kBlk + 1], kq[kBlk][kBlk + 1], lw[4][kBlk][kBlk + 1];
     const int blk = blockIdx.x, kh = blockIdx.y, lane = threadIdx.x, n_k = a.n_k, n_v = a.n_v, group = n_v / n_k;
@@ -171,7 +189,7 @@ __global__ __launch_bounds__(64) void dn_block_kernel(DnPrefillArgs a, int M) {
 #pragma unroll
             for (int j = 0; j < b; ++j) v = fmaf(-lw[g][b][j], tcol[j], v);
             tcol[b] = v;
-            if (live) out->tb[b][c] = v * beta_c;
+            if (live) out->tb[b][c] = b >= c ? v * beta_c : 0.0f;  // (0 also where a later token's beta is NaN)
         }
         __syncthreads();
     }
@@ -270,7 +288,7 @@ __global__ __launch_bounds__(kThreads) void dn_recur_kernel(DnPrefillArgs a, int
         const float gv[4] = {d.g.x, d.g.y, d.g.z, d.g.w}, pl[4] = {d.pl.x, d.pl.y, d.pl.z, d.pl.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) z[i] = d.v[i] - gv[i] * z[i];
-        const f32x4_t u = mfma16(d.tb, as_float4(z), f32x4_t{});
+        const f32x4_t u = lower16(d.tb, z, f32x4_t{}, g);
         f32x4_t pu;
 #pragma unroll
         for (int i = 0; i < 4; ++i) pu[i] = pl[i] * u[i];
@@ -283,7 +301,7 @@ __global__ __launch_bounds__(kThreads) void dn_recur_kernel(DnPrefillArgs a, int
             for (int w = 1; w < kWaves; ++w) o = o + part[par][1][w][lane];
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[i] = gv[i] * o[i];
-            o = mfma16(d.a, as_float4(u), o);
+            o = lower16(d.a, u, o, g);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int m = blk * kBlk + 4 * g + i;

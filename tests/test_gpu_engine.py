@@ -510,6 +510,58 @@ def test_prefill_recurrence_blocks(snl_mod, rows):
         e.close()
 
 
+@pytest.fixture(scope="module")
+def overflowing(snl_mod, tmp_path_factory):
+    """A model of DeltaNet layers whose embedding of token 7 overflows (block scales of 3e38), from a file."""
+    import dataclasses
+
+    import snl_format as F
+
+    cfg = dataclasses.replace(snl_mod.tiny_config(), full_attention=[False] * 8, mhc=None, has_mtp=False)
+    e = snl_mod.Engine(cfg, seed=41, quant=0, ctx=64)
+    path = str(tmp_path_factory.mktemp("overflow") / "model.snl")
+    e.save(path, None, model_name="overflow")
+    e.close()
+    header, tensors, _ = F.read(path)
+    items = []
+    for name in sorted(header["tensors"], key=lambda n: header["tensors"][n]["offset"]):
+        dtype, shape, q, sc = tensors[name]
+        if name == "embed":
+            sc = sc.copy().reshape(cfg.vocab, -1)
+            sc[7] = 3e38
+            sc = sc.reshape(-1)
+        items.append((name, dtype, tuple(shape), q.tobytes(), sc))
+    F.write(path, "overflow", header["quant"], header["config"], items)
+    e = snl_mod.Engine.load(path, None, ctx=64)
+    yield cfg, e
+    e.close()
+
+
+@pytest.mark.parametrize("rows,bad", [(3, 2), (10, 9), (16, 2), (16, 15), (17, 16), (19, 18), (26, 9), (33, 32)])
+def test_prefill_later_token_not_finite(overflowing, rows, bad):
+    """A token whose rows are not finite leaves the tokens before it as they were, bit for bit, wherever it
+    stands in a block of the recurrence: the pass's first two hidden rows and its second-last logits row."""
+    cfg, e = overflowing
+    print(f"not finite: {rows} rows, token {bad}", flush=True)
+    prompt = [t if t != 7 else 8 for t in _prompt(20 + rows, cfg.vocab, seed=rows)]
+    pos = [[i] * 3 for i in range(20 + rows)]
+
+    def run(tokens):
+        e.reset()
+        e.forward(tokens[:20], pos[:20])
+        lg, _ = e.forward(tokens[20:], pos[20:], logit_rows=2)
+        return lg, e.buffer(1).reshape(3, cfg.hidden)[1:]
+
+    lg, hid = run(prompt)
+    assert np.isfinite(lg).all() and np.isfinite(hid).all()
+    lg_b, hid_b = run(prompt[:20 + bad] + [7] + prompt[21 + bad:])
+    assert not np.isfinite(lg_b[1]).any()
+    n = min(2, bad)
+    assert np.array_equal(hid_b[:n], hid[:n])
+    if bad == rows - 1:
+        assert np.array_equal(lg_b[0], lg[0])
+
+
 @pytest.mark.parametrize("n", [512, 1024])
 def test_draft_after_full_prefill_chunk(snl_mod, oracle, n):
     """A prompt whose last prefill pass is a full 512 rows leaves the first draft at hidden row 512;
