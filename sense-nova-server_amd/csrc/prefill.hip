@@ -124,18 +124,22 @@ __device__ __forceinline__ float4 as_float4(f32x4_t v) { return make_float4(v[0]
 
 // acc + L X of a lower triangular L (lv: columns 4g .. 4g + 3 of row l % 16) and X in accumulator layout
 // (row 4g + i).  The product adds 0 x the rows past a row's own, which is NaN where such a row is not
-// finite: then each row is formed with those rows taken as 0, so a token never sees a later one.
+// finite: then each row is formed again with those rows taken as 0, so a token never sees a later one.
+// (The check runs beside the product's MFMAs: 512 tokens of 32 heads, the conv included, 94 us without it,
+// 104 with it made before them and the 16 rows unrolled, 93 so.)
 __device__ __forceinline__ f32x4_t lower16(const float4& lv, f32x4_t x, f32x4_t acc, int g) {
+    f32x4_t out = mfma16(lv, as_float4(x), acc);
     const float mag = (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3]));
-    if (!__any(!(mag < INFINITY))) return mfma16(lv, as_float4(x), acc);
-    f32x4_t out = {};
-    for (int b = 0; b < 16; ++b) {
-        f32x4_t xb;
+    if (__any(!(mag < INFINITY))) {
+#pragma unroll 1
+        for (int b = 0; b < 16; ++b) {
+            f32x4_t xb;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) xb[i] = 4 * g + i <= b ? x[i] : 0.0f;
-        const f32x4_t y = mfma16(lv, as_float4(xb), acc);
+            for (int i = 0; i < 4; ++i) xb[i] = 4 * g + i <= b ? x[i] : 0.0f;
+            const f32x4_t y = mfma16(lv, as_float4(xb), acc);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[i] = 4 * g + i == b ? y[i] : out[i];
+            for (int i = 0; i < 4; ++i) out[i] = 4 * g + i == b ? y[i] : out[i];
+        }
     }
     return out;
 }
