@@ -111,6 +111,7 @@ struct DnBlock {  // of one (block, value head)
     float g[kBlk], pl[kBlk];
 };
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 // acc += X Y^T over 16 columns of both: xv / yv hold columns 4g .. 4g + 3 of the lane's row l % 16
 // (v_mfma_f32_16x16x4_f32, the 4 lane groups' g as its K); acc row 4g + i, column l % 16
@@ -122,13 +123,13 @@ __device__ __forceinline__ f32x4_t mfma16(const float4& xv, const float4& yv, f3
 }
 __device__ __forceinline__ float4 as_float4(f32x4_t v) { return make_float4(v[0], v[1], v[2], v[3]); }
 
-// acc + L X of a lower triangular L (lv: columns 4g .. 4g + 3 of row l % 16) and X in accumulator layout
+// L X of a lower triangular L (lv: columns 4g .. 4g + 3 of row l % 16) and X in accumulator layout
 // (row 4g + i).  The product adds 0 x the rows past a row's own, which is NaN where such a row is not
 // finite: then each row is formed again with those rows taken as 0, so a token never sees a later one.
 // (The check runs beside the product's MFMAs: 512 tokens of 32 heads, the conv included, 94 us without it,
 // 104 with it made before them and the 16 rows unrolled, 93 so.)
-__device__ __forceinline__ f32x4_t lower16(const float4& lv, f32x4_t x, f32x4_t acc, int g) {
-    f32x4_t out = mfma16(lv, as_float4(x), acc);
+__device__ __forceinline__ f32x4_t lower16(const float4& lv, f32x4_t x, int g) {
+    f32x4_t out = mfma16(lv, as_float4(x), f32x4_t{});
     const float mag = (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3]));
     if (__any(!(mag < INFINITY))) {
 #pragma unroll 1
@@ -136,7 +137,7 @@ __device__ __forceinline__ f32x4_t lower16(const float4& lv, f32x4_t x, f32x4_t 
             f32x4_t xb;
 #pragma unroll
             for (int i = 0; i < 4; ++i) xb[i] = 4 * g + i <= b ? x[i] : 0.0f;
-            const f32x4_t y = mfma16(lv, as_float4(xb), acc);
+            const f32x4_t y = mfma16(lv, as_float4(xb), f32x4_t{});
 #pragma unroll
             for (int i = 0; i < 4; ++i) out[i] = 4 * g + i == b ? y[i] : out[i];
         }
@@ -151,17 +152,23 @@ __global__ __launch_bounds__(64) void dn_block_kernel(DnPrefillArgs a, int M) {
     const int t = blk * kBlk + c;
     const float4* kp = reinterpret_cast<const float4*>(a.k + ((size_t)min(t, M - 1) * n_k + kh) * DK) + g;
     const float4* qp = reinterpret_cast<const float4*>(a.q + ((size_t)min(t, M - 1) * n_k + kh) * DK) + g;
-    f32x4_t dk = {}, dq = {};
+    // In 64 bits: the deltas take differences of rows that are alike, so what rounding leaves in k . k and
+    // q . k comes back enlarged (v_mfma_f64_16x16x4_f64: row 4i + g, column l % 16; see dn_recur_kernel)
+    f64x4_t dk = {}, dq = {};
 #pragma unroll
     for (int s = 0; s < DK / 16; ++s) {
         const float4 k4 = kp[4 * s], q4 = qp[4 * s];
-        dk = mfma16(k4, k4, dk);
-        dq = mfma16(q4, k4, dq);
+        const float kv[4] = {k4.x, k4.y, k4.z, k4.w}, qv[4] = {q4.x, q4.y, q4.z, q4.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            dk = __builtin_amdgcn_mfma_f64_16x16x4f64((double)kv[i], (double)kv[i], dk, 0, 0, 0);
+            dq = __builtin_amdgcn_mfma_f64_16x16x4f64((double)qv[i], (double)kv[i], dq, 0, 0, 0);
+        }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        kk[4 * g + i][c] = dk[i];  // k_b . k_c
-        kq[4 * g + i][c] = dq[i];  // q_b . k_c
+        kk[4 * i + g][c] = (float)dk[i];  // k_b . k_c
+        kq[4 * i + g][c] = (float)dq[i];  // q_b . k_c
     }
     __syncthreads();
     // lane group g takes value heads g, g + 4, ... of the key head, lane c column c of its matrices
@@ -223,6 +230,11 @@ __global__ __launch_bounds__(256) void dn_conv_state_kernel(DnPrefillArgs a, int
 // What bounds it: the chain through a block (two products, an exchange between the waves and another
 // product, 1.6 us per 16 tokens).  512 tokens of 32 heads take 52 us + 7.5 in dn_block_kernel; on the
 // vector ALUs, 4 tokens at a time with every row sum reduced across lanes, they took 154 + 5.
+// Rounding: each wave's products are sums of 16 from zero, added in pairs, then to the decayed state or the
+// value in one fma.  Against 64 bits (17 / 512 tokens, error of the outputs, decays near 1): 1.1e-7 / 2.0e-7;
+// with k . k as one f32 sum of 128 and the state as accumulator of its products 1.7e-7 / 2.9e-7, and
+// 2.7e-7 / 3.1e-7 against 1.3e-7 / 1.6e-7 where keys are alike; token by token in blocks of 4 on the vector
+// ALUs 1.3e-7 / 2.8e-7 and 1.0e-7 / 1.5e-7.  The time is the same.
 struct RecurIn {
     float4 k[2], q[2];   // token l % 16, rows 32w + 16t + 4g ..
     float kt[2][4];      // token 4g + i, row 32w + 16t + l % 16
@@ -275,37 +287,40 @@ __global__ __launch_bounds__(kThreads) void dn_recur_kernel(DnPrefillArgs a, int
         d.pl = reinterpret_cast<const float4*>(b->pl)[g];
         d.glast = b->g[kBlk - 1];
     };
+    auto wave_parts = [&](int par, int which) {  // the waves' shares of a product, added in pairs
+        const auto& p = part[par][which];
+        return (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]);
+    };
     auto step = [&](int blk, const RecurIn& d) {
         const int par = blk & 1;
-        f32x4_t ks = {}, qs = {};
+        f32x4_t ks[2], qs[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) ks = mfma16(d.k[t], as_float4(s[t]), ks);
+        for (int t = 0; t < 2; ++t) ks[t] = mfma16(d.k[t], as_float4(s[t]), f32x4_t{});
 #pragma unroll
-        for (int t = 0; t < 2; ++t) qs = mfma16(d.q[t], as_float4(s[t]), qs);
-        part[par][0][wave][lane] = ks;
-        part[par][1][wave][lane] = qs;
+        for (int t = 0; t < 2; ++t) qs[t] = mfma16(d.q[t], as_float4(s[t]), f32x4_t{});
+        part[par][0][wave][lane] = ks[0] + ks[1];
+        part[par][1][wave][lane] = qs[0] + qs[1];
         // (one barrier a block: the other parity's sums are read before the next one)
         __syncthreads();
-        f32x4_t z = part[par][0][0][lane];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) z = z + part[par][0][w][lane];
+        f32x4_t z = wave_parts(par, 0);
         const float gv[4] = {d.g.x, d.g.y, d.g.z, d.g.w}, pl[4] = {d.pl.x, d.pl.y, d.pl.z, d.pl.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) z[i] = d.v[i] - gv[i] * z[i];
-        const f32x4_t u = lower16(d.tb, z, f32x4_t{}, g);
+        for (int i = 0; i < 4; ++i) z[i] = fmaf(-gv[i], z[i], d.v[i]);
+        const f32x4_t u = lower16(d.tb, z, g);
         f32x4_t pu;
 #pragma unroll
         for (int i = 0; i < 4; ++i) pu[i] = pl[i] * u[i];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-            s[t] = mfma16(make_float4(d.kt[t][0], d.kt[t][1], d.kt[t][2], d.kt[t][3]), as_float4(pu), s[t] * d.glast);
+        for (int t = 0; t < 2; ++t) {
+            const f32x4_t ku = mfma16(make_float4(d.kt[t][0], d.kt[t][1], d.kt[t][2], d.kt[t][3]), as_float4(pu), f32x4_t{});
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[t][i] = fmaf(d.glast, s[t][i], ku[i]);
+        }
         if (wave == (blk & (kWaves - 1))) {  // the outputs: the waves take turns
-            f32x4_t o = part[par][1][0][lane];
+            f32x4_t o = wave_parts(par, 1);
+            const f32x4_t au = lower16(d.a, u, g);
 #pragma unroll
-            for (int w = 1; w < kWaves; ++w) o = o + part[par][1][w][lane];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = gv[i] * o[i];
-            o = lower16(d.a, u, o, g);
+            for (int i = 0; i < 4; ++i) o[i] = fmaf(gv[i], o[i], au[i]);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int m = blk * kBlk + 4 * g + i;
