@@ -6,8 +6,7 @@
 // cache at the token's cache position.
 //
 // attend: block (kv head, 16 queries, key part), wave w = query head 4*kv + w of the GQA group;
-// the block streams its part of the keys [0, last query's position] (128 to 4096 keys, part_keys) in
-// steps of 32 through LDS (K rows and V rows, each staged with 16-byte copies; the V^T fragments come
+// the block streams its part of the keys [0, last query's position] in steps of 32 through LDS (K rows and V rows, each staged with 16-byte copies; the V^T fragments come
 // back from the V rows through the transposing LDS read, two 8-byte reads per fragment),
 // shared by the group's 4 heads.
 //   scores  S^T = K Q^T on v_mfma_f32_16x16x32_f16: A = 16 keys x 32 dims of K (exact f16),
@@ -18,9 +17,14 @@
 //           position weigh 0;
 //   values  O^T += V^T P^T: B = the lane's own 8 probabilities as f16 hi + lo (keys 4g..4g+3 and
 //           16+4g..16+4g+3, the same order in the V^T fragment), A = 16 dims x those keys.
-// With one part the output is divided by the softmax sum and multiplied by the sigmoid gate, as in
-// combine; with several, each part leaves (unnormalised output, running max, sum) and
-// pf_combine_kernel merges the parts in order.
+//
+// A query's keys are summed the same way whatever shares its pass: every leaf of 256 keys (128 within the
+// cache's first 512) from zero, the leaves of 1024 keys to a node, two nodes to a top and the tops one
+// after the other, each time merged in order (merge()).  A part is a leaf, a node or a top (part_level),
+// so a block merges what lies inside its part and pf_combine_kernel the rest, by the same steps; a leaf
+// past a query's position weighs 0 and changes nothing.  Each part leaves (unnormalised output, running max,
+// sum); with one part the output is divided by the softmax sum and multiplied by the sigmoid gate at
+// once, as in combine.
 #include <float.h>
 
 #include <algorithm>
@@ -37,8 +41,11 @@ namespace {
 
 constexpr int HD = 256, G = 4;
 constexpr int QTILE = 16, KB = 32;
-constexpr int KPART = 4096, KPART_MIN = 128;  // most and fewest keys of a part
-constexpr int kBlocks = 512;                   // blocks a launch aims at
+// Keys summed from zero, and merged.  The first 512 keys have shorter leaves, for the short contexts whose
+// blocks are few: 45 rows over 260 keys 32 us a launch in leaves of 256, 25 in leaves of 128.
+constexpr int LEAF = 256, FINE = 128, FINE_KEYS = 512, NODE = 1024, TOP = 2 * NODE;
+constexpr int kNodeLeaves = NODE / LEAF, kFirstLeaves = kNodeLeaves + FINE_KEYS / FINE - FINE_KEYS / LEAF;
+constexpr int PSTRIDE = HD + 4;  // floats of a part's partial: output, running max, sum (16-byte rows)
 constexpr int KROW = HD + 8;  // K tile row (halfs): 528 bytes keeps the 16 rows of a read on distinct banks
 constexpr int VROW = HD + 16;  // V row (halfs): 544 bytes, so the 4 rows of a transposed read hit distinct banks
 
@@ -46,6 +53,31 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// the weights of two partials with running maxima ma and mb in their merge (one of them is 1); ma becomes
+// the merge's
+__device__ __forceinline__ void merge_weights(float& ma, float mb, float& fa, float& fb) {
+    const float e = expf(-fabsf(ma - mb));
+    fa = ma >= mb ? 1.0f : e;
+    fb = ma >= mb ? e : 1.0f;
+    ma = fmaxf(ma, mb);
+}
+__device__ __forceinline__ float merge(float a, float fa, float b, float fb) { return fmaf(b, fb, a * fa); }
+__device__ __forceinline__ f32x4_t merge4(f32x4_t a, float fa, f32x4_t b, float fb) {
+    return f32x4_t{merge(a[0], fa, b[0], fb), merge(a[1], fa, b[1], fb), merge(a[2], fa, b[2], fb),
+                   merge(a[3], fa, b[3], fb)};
+}
+
+// the first key of part p, and the parts of `keys` keys, where a part is a leaf, a node or a top
+__host__ __device__ constexpr int part_key(int level, int p) {
+    if (level) return p * (level > 1 ? TOP : NODE);
+    return p < FINE_KEYS / FINE ? p * FINE : FINE_KEYS + (p - FINE_KEYS / FINE) * LEAF;
+}
+__host__ __device__ constexpr int part_count(int level, int keys) {
+    if (level) return (keys + (level > 1 ? TOP : NODE) - 1) / (level > 1 ? TOP : NODE);
+    return keys <= FINE_KEYS ? (keys + FINE - 1) / FINE : FINE_KEYS / FINE + (keys - FINE_KEYS + LEAF - 1) / LEAF;
+}
+__device__ __forceinline__ int leaf_end(int key) { return key + (key < FINE_KEYS ? FINE : LEAF); }
 
 __global__ __launch_bounds__(256) void pf_prep_kernel(AttnArgs a, const PrefillDev* st) {
     __shared__ float sh[HD];
@@ -86,18 +118,23 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(AttnArgs a, const PrefillD
     }
 }
 
-__global__ __launch_bounds__(256, 2) void pf_attend_kernel(AttnArgs a, const PrefillDev* st, int M, float* part,
-                                                        int parts, int kpart) {
+// A node's sums stay beside the leaf's: NR of its 16 output tiles in registers, the others in LDS, as much
+// of each as two blocks on a CU have.  A top's first node waits in the block's own partial.
+template <int LEVEL>
+__global__ __launch_bounds__(256, 2) void pf_attend_kernel(AttnArgs a, const PrefillDev* st, int M, int row0, float* part,
+                                                           int parts) {
+    constexpr int NR = LEVEL ? 5 : 0;
+    __shared__ __align__(16) f32x4_t node_lds[LEVEL ? 16 - NR : 1][LEVEL ? 256 : 1];
     __shared__ __align__(16) _Float16 ks[KB * KROW];
     __shared__ __align__(16) _Float16 vs[KB * VROW];
-    const int kh = blockIdx.x, q0 = blockIdx.y * QTILE;
+    const int kh = blockIdx.x, q0 = row0 + blockIdx.y * QTILE;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hh = kh * G + w;
     const int pos0 = st->pos0;
     const int qn = min(QTILE, M - q0);
     const int kend = pos0 + q0 + qn;  // keys of the block's last query
     const int p = blockIdx.z;
-    const int kfirst = p * kpart, kstop = min(kend, kfirst + kpart);
+    const int kfirst = part_key(LEVEL, p), kstop = min(kend, part_key(LEVEL, p + 1));
     if (kfirst >= kend) return;
     const int q_dim = a.n_heads * HD, kv_dim = a.n_kv * HD;
     const int j = lane & 15, g = lane >> 4;
@@ -135,9 +172,12 @@ __global__ __launch_bounds__(256, 2) void pf_attend_kernel(AttnArgs a, const Pre
         }
 
     f32x4_t o[16];
-#pragma unroll
-    for (int dt = 0; dt < 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float mrun = -1e30f, lpart = 0.0f;
+    float mrun, lpart, l;
+    f32x4_t node[NR ? NR : 1];
+    float node_m = 0.0f, node_l = 0.0f, top_m = 0.0f, top_l = 0.0f;
+    // (lanes past the pass's rows read the first row's partial and write none)
+    float* pp = part + (((size_t)((qvalid ? mq : q0) - row0) * a.n_heads + hh) * parts + p) * PSTRIDE;
+    f32x4_t* prow = reinterpret_cast<f32x4_t*>(pp + 4 * g);  // this lane's 16 bytes of output tile dt at prow[4 dt]
     const uint16_t* kc = a.kcache + kh * HD;
     const uint16_t* vc = a.vcache + kh * HD;
 
@@ -158,7 +198,7 @@ __global__ __launch_bounds__(256, 2) void pf_attend_kernel(AttnArgs a, const Pre
         }
     };
     load_rows(kfirst);
-    for (int kb = kfirst; kb < kstop; kb += KB) {
+    auto step = [&](int kb) {
         __syncthreads();  // the previous step's tiles are consumed
         {
             const int key = tid >> 3, seg = tid & 7;
@@ -231,16 +271,59 @@ __global__ __launch_bounds__(256, 2) void pf_attend_kernel(AttnArgs a, const Pre
             o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, o[dt], 0, 0, 0);
             o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, o[dt], 0, 0, 0);
         }
+    };
+    for (int kn = kfirst; kn < kstop; kn += NODE) {
+        const int nstop = min(kstop, kn + NODE);
+        for (int kl = kn; kl < nstop; kl = leaf_end(kl)) {
+#pragma unroll
+            for (int dt = 0; dt < 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            mrun = -1e30f;
+            lpart = 0.0f;
+            for (int kb = kl; kb < min(nstop, leaf_end(kl)); kb += KB) step(kb);
+            l = xor_sum<32>(xor_sum<16>(lpart));
+            if constexpr (LEVEL > 0) {  // o, mrun, l: the node's sums up to this leaf
+                if (kl > kn) {
+                    float fa, fb;
+                    merge_weights(node_m, mrun, fa, fb);
+                    mrun = node_m;
+                    l = merge(node_l, fa, l, fb);
+#pragma unroll
+                    for (int dt = 0; dt < 16; ++dt)
+                        o[dt] = merge4(dt < NR ? node[dt < NR ? dt : 0] : node_lds[dt < NR ? 0 : dt - NR][tid], fa, o[dt], fb);
+                }
+                if (leaf_end(kl) < nstop) {
+                    node_m = mrun;
+                    node_l = l;
+#pragma unroll
+                    for (int dt = 0; dt < 16; ++dt) {
+                        if (dt < NR) node[dt < NR ? dt : 0] = o[dt];
+                        else node_lds[dt < NR ? 0 : dt - NR][tid] = o[dt];
+                    }
+                }
+            }
+        }
+        if constexpr (LEVEL > 1) {
+            if (kn > kfirst) {
+                float fa, fb;
+                merge_weights(top_m, mrun, fa, fb);
+                mrun = top_m;
+                l = merge(top_l, fa, l, fb);
+#pragma unroll
+                for (int dt = 0; dt < 16; ++dt) o[dt] = merge4(prow[4 * dt], fa, o[dt], fb);
+            } else if (nstop < kstop) {
+                top_m = mrun;
+                top_l = l;
+                if (qvalid)
+#pragma unroll
+                    for (int dt = 0; dt < 16; ++dt) prow[4 * dt] = o[dt];
+            }
+        }
     }
     // ---- normalise, gate, store: lane (query j) holds dims 16dt + 4g + r ----
-    const float l = xor_sum<32>(xor_sum<16>(lpart));
     if (!qvalid) return;
     if (parts > 1) {  // this part's unnormalised output, running max and sum for the combine
-        float* pp = part + (((size_t)mq * a.n_heads + hh) * parts + p) * (HD + 2);
 #pragma unroll
-        for (int dt = 0; dt < 16; ++dt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) pp[16 * dt + 4 * g + r] = o[dt][r];
+        for (int dt = 0; dt < 16; ++dt) prow[4 * dt] = o[dt];
         if (g == 0) {
             pp[HD] = mrun;
             pp[HD + 1] = l;
@@ -258,64 +341,127 @@ __global__ __launch_bounds__(256, 2) void pf_attend_kernel(AttnArgs a, const Pre
         }
 }
 
-// Merge the key parts of one (query, head): block (head, query), thread = dim.  Parts are added
-// in order with weights e^(m_p - max); then the division by the softmax sum and the sigmoid gate.
-__global__ __launch_bounds__(HD) void pf_combine_kernel(AttnArgs a, const PrefillDev* st, int M, const float* part,
-                                                        int parts, int kpart) {
-    const int hh = blockIdx.x, m = blockIdx.y, d = threadIdx.x;
-    const int q0 = m / QTILE * QTILE, qn = min(QTILE, M - q0);
-    const int nparts = (st->pos0 + q0 + qn + kpart - 1) / kpart;
-    const float* pp = part + ((size_t)m * a.n_heads + hh) * parts * (HD + 2);
-    float mx = -1e30f;
-    for (int p = 0; p < nparts; ++p) mx = fmaxf(mx, pp[(size_t)p * (HD + 2) + HD]);
-    float acc = 0.0f, l = 0.0f;
-    for (int p = 0; p < nparts; ++p) {
-        const float* q = pp + (size_t)p * (HD + 2);
-        const float f = expf(q[HD] - mx);
-        acc = acc + q[d] * f;
-        l = l + q[HD + 1] * f;
+// Merge the key parts of one (query, head): block (4 heads, query), a wave per head, lane = 4 dims.  Parts
+// of a node, nodes of a top, then the tops, each in order; then the division by the softmax sum and the
+// sigmoid gate.
+struct Partial {
+    f32x4_t o;
+    float m, l;
+    __device__ __forceinline__ void add(const Partial& b, bool first) {
+        if (first) {
+            *this = b;
+            return;
+        }
+        float fa, fb;
+        merge_weights(m, b.m, fa, fb);
+        o = merge4(o, fa, b.o, fb);
+        l = merge(l, fa, b.l, fb);
     }
-    const float gate = a.proj[(size_t)m * a.proj_stride + hh * 2 * HD + HD + d];
-    a.out[(size_t)m * a.n_heads * HD + hh * HD + d] = acc / l / (1.0f + expf(-gate));
+};
+
+template <int LEVEL>
+__global__ __launch_bounds__(256) void pf_combine_kernel(AttnArgs a, const PrefillDev* st, int M, int row0,
+                                                         const float* part, int parts) {
+    const int hh = blockIdx.x * G + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int m = row0 + blockIdx.y, q0 = m / QTILE * QTILE, qn = min(QTILE, M - q0);
+    const int nparts = part_count(LEVEL, st->pos0 + q0 + qn);
+    const float* pp = part + ((size_t)blockIdx.y * a.n_heads + hh) * parts * PSTRIDE + 4 * lane;
+    const float* ml = pp - 4 * lane + HD;
+    Partial tot = {}, top = {};
+    for (int p = 0, n = 0; p < nparts; ++n) {
+        // node n's partial: of its parts (leaves, the first node's first ones shorter), or itself
+        Partial node = {};
+        if constexpr (LEVEL == 0) {
+            Partial in[kFirstLeaves];
+            const int count = min(n ? kNodeLeaves : kFirstLeaves, nparts - p);
+#pragma unroll
+            for (int i = 0; i < kFirstLeaves; ++i) {
+                const size_t at = (size_t)min(p + i, nparts - 1) * PSTRIDE;
+                in[i] = Partial{*reinterpret_cast<const f32x4_t*>(pp + at), ml[at], ml[at + 1]};
+            }
+#pragma unroll
+            for (int i = 0; i < kFirstLeaves; ++i)
+                if (i < count) node.add(in[i], i == 0);
+            p += count;
+        } else {
+            const size_t at = (size_t)p * PSTRIDE;
+            node = Partial{*reinterpret_cast<const f32x4_t*>(pp + at), ml[at], ml[at + 1]};
+            ++p;
+        }
+        const bool top_first = LEVEL > 1 || n % (TOP / NODE) == 0;
+        top.add(node, top_first);
+        if (LEVEL > 1 || n % (TOP / NODE) == TOP / NODE - 1 || p >= nparts) tot.add(top, n < TOP / NODE && (LEVEL < 2 || n == 0));
+    }
+    const float* grow = a.proj + (size_t)m * a.proj_stride + hh * 2 * HD + HD + 4 * lane;
+    float* orow = a.out + ((size_t)m * a.n_heads + hh) * HD + 4 * lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) orow[r] = tot.o[r] / tot.l / (1.0f + expf(-grow[r]));
 }
 
 }  // namespace
 
-// Keys per part of a pass over `keys` keys: as many parts as give the chip kBlocks blocks (two fit a
-// CU), of at least KPART_MIN keys, and no part longer than KPART.  A step of 32 keys is a chain of
-// loads, LDS and dependent MFMAs that one block alone takes 3.3 us for, so few blocks of many steps
-// leave the chip idle: 16 heads, 45 rows over 1045 keys 109 us in 12 blocks, 18 + 9 (combine) in 108;
-// 512 rows over 1000 keys 83 us in 128 blocks, 28 + 15 in 512; 512 rows at 12800 keys 382 us in parts
-// of 4096, 192 + 17 in four of 3200 (both also with the next step's rows loaded ahead).
-static int part_keys(int M, int n_kv, int keys) {
-    const int base = n_kv * ((M + QTILE - 1) / QTILE);
-    const int parts = std::max(1, kBlocks / base);
-    return std::min(KPART, std::max(KPART_MIN, ((keys + parts - 1) / parts + KB - 1) / KB * KB));
+static int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+// The level of the parts of a pass over `keys` keys.  A step of 32 keys is a chain of loads, LDS and dependent
+// MFMAs that one block alone takes 3.3 us for, so few blocks of many steps leave the chip idle (two fit a CU);
+// past two rounds of leaves their partials cost more than longer blocks do.  us a call in parts of a leaf /
+// node / top, 16 heads: 512 rows over 2048 keys 98 / 101 / 175 (1024 blocks of a leaf), 4600 200 / 157 / 176,
+// 12800 495 / 342 / 355 (1664 blocks of a node), 32768 1336 / 837 / 796; 100 rows over 7000 keys 74 / 88 / 156,
+// 9500 102 / 94 / 157; 45 rows over 12800 keys 76 / 88 / 156.
+// Parts of any length, cut by the blocks that a pass gives, were faster where rows are many (512 rows over
+// 1000 keys 69 us, 72 so; 12800 314 and 345; 45 rows over 1045 30 and 35) and slower where they are few (3 over
+// 12800 74 and 48), but a token's sums then changed with the tokens that shared its pass.
+// A launch takes as many query tiles as keep its partials within kMaxBlocks blocks' (136 MB, 16 heads at any
+// context).
+constexpr int kLeafBlocks = 1024, kMaxBlocks = 2048;
+static int part_level(int tiles, int n_kv, int keys) {
+    if (keys <= FINE || n_kv * tiles * part_count(0, keys) <= kLeafBlocks) return 0;
+    return keys <= NODE || n_kv * tiles * part_count(1, keys) <= kMaxBlocks ? 1 : 2;
+}
+static int launch_tiles(int tiles, int n_kv, int parts) {
+    const int most = std::max(1, kMaxBlocks / (n_kv * parts));
+    return cdiv(tiles, cdiv(tiles, most));
 }
 
 size_t attention_prefill_part_floats(int ctx, int n_heads) {
-    if (ctx <= KPART_MIN || n_heads < G) return 0;  // one part, or a model without attention
+    if (ctx <= FINE || n_heads < G) return 0;  // one part, or a model without attention
+    const int n_kv = n_heads / G;
     size_t most = 0;
-    for (int m = QTILE; m <= SNL_PF_M; m += QTILE) {
-        const int kp = part_keys(m, n_heads / G, ctx);
-        // a shorter context has shorter parts, so no more of them than kBlocks / base or ctx / KPART
-        const size_t parts = std::max<size_t>((ctx + kp - 1) / kp, std::min(kBlocks / (n_heads / G * (m / QTILE)), ctx / KPART_MIN + 1));
-        most = std::max(most, (size_t)m * n_heads * (parts + 1) * (HD + 2));
+    for (int tiles = 1; tiles <= SNL_PF_M / QTILE; ++tiles) {
+        // of any pass up to ctx positions: as many parts as each level's blocks, or its keys, allow
+        const int base = n_kv * tiles;
+        const int parts[3] = {std::min(part_count(0, ctx), kLeafBlocks / base),
+                              std::min(part_count(1, ctx), std::max(1, kMaxBlocks / base)), part_count(2, ctx)};
+        for (int n : parts)
+            most = std::max(most, std::min((size_t)base * n, (size_t)std::max(kMaxBlocks, n_kv * n)));
     }
-    return most;
+    return most * QTILE * G * PSTRIDE;
+}
+
+template <int LEVEL>
+static void launch_parts(const AttnArgs& a, const PrefillDev* pstep, int M, float* part, int parts, int tiles,
+                         hipStream_t s) {
+    for (int row0 = 0; row0 < M; row0 += tiles * QTILE) {
+        const int rows = std::min(M - row0, tiles * QTILE);
+        hipLaunchKernelGGL(pf_attend_kernel<LEVEL>, dim3(a.n_kv, cdiv(rows, QTILE), parts), dim3(256), 0, s, a, pstep, M,
+                           row0, part, parts);
+        if (parts > 1)
+            hipLaunchKernelGGL(pf_combine_kernel<LEVEL>, dim3(a.n_kv, rows), dim3(256), 0, s, a, pstep, M, row0, part,
+                               parts);
+    }
 }
 
 int launch_attention_prefill(const AttnArgs& a, const PrefillDev* pstep, int M, int keys, float* part,
                              size_t part_floats, hipStream_t s) {
     if (M < 1 || M > SNL_PF_M || a.n_kv < 1 || a.n_heads != G * a.n_kv || a.rot_dim > HD || a.rot_dim % 2 || !pstep) return -1;
-    const int kpart = part_keys(M, a.n_kv, keys);
-    const int parts = (keys + kpart - 1) / kpart;  // parts of the pass's longest key range
-    if (parts > 1 && (!part || (size_t)M * a.n_heads * parts * (HD + 2) > part_floats)) return -1;
+    const int tiles = cdiv(M, QTILE), level = part_level(tiles, a.n_kv, keys);
+    const int parts = part_count(level, keys);  // parts of the pass's longest key range
+    const int step = launch_tiles(tiles, a.n_kv, parts);
+    if ((parts > 1 || level > 1) && (!part || (size_t)step * QTILE * a.n_heads * parts * PSTRIDE > part_floats)) return -1;
     hipLaunchKernelGGL(pf_prep_kernel, dim3(a.n_heads + 2 * a.n_kv, M), dim3(256), 0, s, a, pstep);
-    hipLaunchKernelGGL(pf_attend_kernel, dim3(a.n_kv, (M + QTILE - 1) / QTILE, parts), dim3(256), 0, s, a, pstep, M,
-                       part, parts, kpart);
-    if (parts > 1)
-        hipLaunchKernelGGL(pf_combine_kernel, dim3(a.n_heads, M), dim3(HD), 0, s, a, pstep, M, part, parts, kpart);
+    if (level == 0) launch_parts<0>(a, pstep, M, part, parts, step, s);
+    else if (level == 1) launch_parts<1>(a, pstep, M, part, parts, step, s);
+    else launch_parts<2>(a, pstep, M, part, parts, step, s);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

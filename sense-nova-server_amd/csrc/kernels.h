@@ -276,8 +276,9 @@ constexpr int kAttnMaxParts = kMaxCtx / kAttnPart;
 // with rotary positions rpos[m]; q/k norm + RoPE, K/V into the f16 cache, then causal
 // attention over every earlier key and the sigmoid gate.  Same AttnArgs, with `pstep` for the
 // positions (step is unused).  keys = pos0 + M (host-side); the key range splits into parts by how
-// many blocks the rows give, whose partials [M][n_heads][parts][258] go to part (part_floats floats;
-// attention_prefill_part_floats is enough for every pass up to ctx positions).
+// many blocks the rows give, whose partials go to part (part_floats floats;
+// attention_prefill_part_floats is enough for every pass up to ctx positions).  A token's results do not
+// depend on the rows that share its pass.
 size_t attention_prefill_part_floats(int ctx, int n_heads);
 int launch_attention_prefill(const AttnArgs& a, const PrefillDev* pstep, int M, int keys, float* part,
                              size_t part_floats, hipStream_t s);

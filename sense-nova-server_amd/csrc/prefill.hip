@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void dn_conv_state_kernel(DnPrefillArgs a, int
 // wave, the state update.  All products run on v_mfma_f32_16x16x4_f32.  A wave reads its own inputs,
 // two blocks ahead of the one computed.
 // What bounds it: the chain through a block (two products, an exchange between the waves and another
-// product, 1.6 us per 16 tokens).  512 tokens of 32 heads take 52 us + 7.5 in dn_block_kernel; on the
+// product, 1.6 us per 16 tokens).  512 tokens of 32 heads take 55 us + 8 in dn_block_kernel; on the
 // vector ALUs, 4 tokens at a time with every row sum reduced across lanes, they took 154 + 5.
 // Rounding: each wave's products are sums of 16 from zero, added in pairs, then to the decayed state or the
 // value in one fma.  Against 64 bits (17 / 512 tokens, error of the outputs, decays near 1): 1.1e-7 / 2.0e-7;

@@ -485,6 +485,73 @@ def test_prefill_attention_key_parts(snl_mod, prefix, rows):
         e.close()
 
 
+@pytest.fixture(scope="module")
+def attention_only(snl_mod):
+    """Engines of two attention layers: 1 KV head (the key parts of a pass are 128 and 256 keys long, from 7936
+    keys of 512 rows on 1024) and 16 KV heads (512 rows: up to 256 keys, then 1024 a part, from 4096 on 2048,
+    and past 8192 keys two launches)."""
+    import dataclasses
+
+    out = {}
+    for n_kv, ctx in ((1, 9800), (16, 8400)):
+        cfg = dataclasses.replace(snl_mod.tiny_config(), n_layers=2, full_attention=[True] * 2, n_heads=4 * n_kv, n_kv_heads=n_kv,
+                                  loop_start=0, loop_end=2, loop_count=1, mhc=None, has_mtp=False)
+        out[n_kv] = cfg, snl_mod.Engine(cfg, seed=23, quant=0, ctx=ctx)
+    yield out
+    for _, e in out.values():
+        e.close()
+
+
+@pytest.mark.parametrize("n_kv,n,splits", [
+    (1, 270, [(270,), (3, 267), (255, 15), (128, 128, 14)]),
+    (1, 1045, [(1000, 45), (1003, 42), (300, 700, 45), (512, 530, 3)]),
+    (1, 9750, [(9216, 534), (9217, 17, 516), (9100, 300, 47, 303)]),
+    (1, 523, [(523,), (509, 14), (512, 8, 3), (384, 139)]),
+    (16, 8300, [(8300,), tuple([48] * 172 + [44]), (1024, 513, 511, 3000, 3252)])])
+def test_prefill_token_independent_of_its_pass(attention_only, n_kv, n, splits):
+    """A token's results do not depend on which tokens share its pass: the last two logits rows of a prompt (which
+    every earlier key enters) are the same bits however it is cut into passes, at each length of key parts."""
+    cfg, e = attention_only[n_kv]
+    prompt = _prompt(n, cfg.vocab, seed=n)
+    pos = [[i] * 3 for i in range(n)]
+    got = []
+    for cut in splits:
+        assert sum(cut) == n
+        print(f"passes of {cut[:6]}", flush=True)
+        e.reset()
+        at = 0
+        for rows in cut:
+            lg, _ = e.forward(prompt[at:at + rows], pos[at:at + rows], logit_rows=2)
+            at += rows
+        got.append(lg)
+    assert np.isfinite(got[0]).all()
+    for lg in got[1:]:
+        assert np.array_equal(lg, got[0])
+
+
+@pytest.mark.parametrize("quant", [0, 1], ids=["q8", "q4"])
+def test_prefill_cut_at_blocks_of_16(snl_mod, quant):
+    """With DeltaNet layers too, whose recurrence takes 16 tokens at a time from a pass's first: a prompt cut at
+    multiples of 16 is the same bits, logits and final DeltaNet state."""
+    cfg = snl_mod.tiny_config()
+    e = snl_mod.Engine(cfg, seed=29, quant=quant, ctx=700)
+    try:
+        prompt = _prompt(667, cfg.vocab, seed=29)
+        pos = [[i] * 3 for i in range(667)]
+        got = []
+        for cut in [(667,), (512, 155), (16, 480, 171), (304, 352, 11)]:
+            e.reset()
+            at = 0
+            for rows in cut:
+                lg, _ = e.forward(prompt[at:at + rows], pos[at:at + rows], logit_rows=2)
+                at += rows
+            got.append((lg, e.buffer(3), e.buffer(4)))
+        for other in got[1:]:
+            assert all(np.array_equal(x, y) for x, y in zip(other, got[0]))
+    finally:
+        e.close()
+
+
 @pytest.mark.parametrize("rows", [3, 15, 16, 17, 32, 33, 49])
 def test_prefill_recurrence_blocks(snl_mod, rows):
     """The DeltaNet recurrence of a prefill pass takes 16 tokens at a time, the last block part full:
