@@ -106,6 +106,8 @@ size_t gemm_s_floats(int N, int K);
 size_t frags_bytes(int M, int K);
 // partial sums that a launch of up to M rows may need
 size_t gemm_part_floats(int M, int N, int K);
+// how a launch with that scratch cuts K: 0 not at all, 1 a block per slice, 2 a block per group of slices
+int gemm_split(int M, int N, int K);
 // reference layout (q [N, K] Q8 / [N, K/2] Q4, s [N, K/32]) -> panel order
 int launch_panel_pack(int quant, int N, int K, const void* q, const float* s, void* qp, float* sp, hipStream_t st);
 int launch_rows_to_frags(const RowsArgs& a, hipStream_t s);

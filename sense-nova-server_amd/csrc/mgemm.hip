@@ -258,23 +258,26 @@ __global__ __launch_bounds__(kRowThreads) void rows_to_frags_kernel(RowsArgs a) 
 // than the stage's products: 64 x 128 blocks 0.98 -> 0.80 us a stage).  The fragments of a block are
 // read from LDS while the block before it is multiplied.
 //
-// What bounds it.  Products alone, with no copy, LDS read or barrier in the loop, take 0.8 of the time
-// (gate_up, 512 rows: 211 of 257 us in 128 x 256 blocks), and those are bound by the matrix cores'
-// rate on real data: the same MFMAs and FMAs in a bare loop run at 2160 TFLOP/s on constant
-// operands and at 1500 on random ones (no instruction waits for another in either).  The hi / lo
-// split doubles the useful flops, so 750 TFLOP/s of a 512-row product is the ceiling of this form.
+// What bounds it.  The same MFMAs and FMAs in a bare loop run at 2160 TFLOP/s on constant operands and at
+// 1500 on random ones (no instruction waits for another in either), the matrix cores' rate on real
+// data.  The hi / lo split doubles the useful flops, so 750 TFLOP/s of a 512-row product is the ceiling
+// of this form.  gate_up at 512 rows reaches 460.  Its products alone, with no copy, LDS read or barrier
+// in the loop, took 211 of 257 us in 128 x 256 blocks, 489 TFLOP/s: 384 blocks are 1.5 rounds of the
+// CUs, and the rest of the distance to 750 is not explained by what was measured.
 //
 // The whole launch, before -> now, Q8 / Q4 (us, N x K, M 512): 24576 x 4096 316 / 301 -> 224 / 223,
 // 12352 x 4096 167 / 196 -> 124 / 126, 4096 x 4096 72 / 65 -> 50 / 51, 4096 x 12288 201 / 183 ->
-// 145 / 141; M 45: 24576 x 4096 69 / 62 -> 44 / 46, 4096 x 4096 64 / 57 -> 16 / 15 and 4096 x 12288
-// 182 / 163 -> 25 / 25, slices split over blocks.
+// 127 / 127 by group (145 / 141 in whole blocks); M 45: 24576 x 4096 69 / 62 -> 44 / 46, 4096 x 4096
+// 64 / 57 -> 16 / 15 and 4096 x 12288 182 / 163 -> 25 / 25, by slice.
 // Slices of K for matrices whose 128-row panels alone leave most CUs idle.  At 4096 x 12288, 45 rows,
-// one block per panel takes 182 us and 8 slices 25; from 46 panels on a split would not pay for its
-// partial sums.  Slices of 512 elements are 8 stages, about as long as a block's first copies take.
+// one block per panel takes 182 us and 8 slices 25.  The line at 46 panels is laid for 512 rows (K 4096:
+// 45 panels in two slices 85 us, 46 in one 73); as a rule on the shape alone it also keeps few rows from a
+// cut that they would gain from (45 rows: 45 panels 17.5 us, 46 39).  Slices of 512 elements are 8 stages,
+// about as long as a block's first copies take.
 constexpr int kSliceMin = 512;
-// 64 x 128 panels up to which a launch splits its slices over blocks (4096 x 4096, 192 rows: 38 us
-// split against 43 whole; 256 rows, 128 panels: whole blocks already fill half the CUs, and the
-// partial sums would be 33 MB)
+// 64 x 128 panels up to which a launch splits its slices over blocks (4096 x 4096: 192 rows, split, 39 us,
+// 193, whole, 44; 4096 x 12288: 72 and, by group, 100; 2048 x 4096: 384 rows 42, 385 44.  More panels were
+// not tried: of 256 rows, 128 panels, the partial sums would be 33 MB)
 constexpr int kSplitPanels = 96;
 
 // WT x WR waves along tokens and rows, TTW x RT 32x32 tiles per wave
@@ -636,22 +639,26 @@ Slices slices_of(int N, int K) {
     return Slices{n, 2 * len, (n + per - 1) / per, per};
 }
 
+// What a block of a launch over several slices runs, where there is scratch for partial sums.
+Split split_of(int M, int N, int K, const Slices& sl) {
+    const int pn = (N + 127) / 128, mtiles = (M + 31) / 32;
+    if (pn * ((mtiles + 1) / 2) <= kSplitPanels) return BY_SLICE;
+    // Many rows: 64 x 128 blocks over all of K, or 128 x 128 ones over a group of slices each, which
+    // read the LDS half as often per product, and kReduce to add the groups' sums.
+    const int whole = xcd_rounds(pn, (mtiles + 1) / 2) * kRoundNarrow * 2;
+    const int by_group = xcd_rounds(pn * sl.groups, (mtiles + 3) / 4) * kRoundMid * 2 / sl.groups;
+    return sl.groups > 1 && by_group * (K / 128) + 2 * kReduce * 32 < whole * (K / 128) ? BY_GROUP : WHOLE;
+}
+
 template <int QT>
 int gemm_dispatch(const GemmArgs& a, hipStream_t s) {
     const int rt = (a.N + 31) / 32, mtiles = (a.M + 31) / 32;
     const Slices sl = slices_of(a.N, a.K);
     if (sl.n > 1) {
-        if (a.part && (rt + 3) / 4 * ((mtiles + 1) / 2) <= kSplitPanels) {
-            if (mtiles <= 1) return gemm_launch<QT, 1, 4, 1, 1, BY_SLICE>(a, 0, rt, sl, s);
-            return gemm_launch<QT, 2, 4, 1, 1, BY_SLICE>(a, 0, rt, sl, s);
-        }
-        // Many rows: 64 x 128 blocks over all of K, or 128 x 128 ones over a group of slices each, which
-        // read the LDS half as often per product, and kReduce to add the groups' sums.
-        const int pn = (rt + 3) / 4;
-        const int whole = xcd_rounds(pn, (mtiles + 1) / 2) * kRoundNarrow * 2;
-        const int by_group = xcd_rounds(pn * sl.groups, (mtiles + 3) / 4) * kRoundMid * 2 / sl.groups;
-        if (a.part && sl.groups > 1 && by_group * (a.K / 128) + 2 * kReduce * 32 < whole * (a.K / 128))
-            return gemm_launch<QT, 2, 4, 2, 1, BY_GROUP>(a, 0, rt, sl, s);
+        const Split split = a.part ? split_of(a.M, a.N, a.K, sl) : WHOLE;
+        if (split == BY_SLICE && mtiles <= 1) return gemm_launch<QT, 1, 4, 1, 1, BY_SLICE>(a, 0, rt, sl, s);
+        if (split == BY_SLICE) return gemm_launch<QT, 2, 4, 1, 1, BY_SLICE>(a, 0, rt, sl, s);
+        if (split == BY_GROUP) return gemm_launch<QT, 2, 4, 2, 1, BY_GROUP>(a, 0, rt, sl, s);
         return gemm_launch<QT, 2, 4, 1, 1, WHOLE>(a, 0, rt, sl, s);
     }
     if (mtiles <= 1) return gemm_launch<QT, 1, 4, 1, 1, WHOLE>(a, 0, rt, sl, s);
@@ -684,6 +691,11 @@ size_t gemm_part_floats(int M, int N, int K) {
     if (sl.n == 1) return 0;
     const int p = (N + 127) / 128;
     return std::max((size_t)sl.n * std::min(M, kSplitPanels / p * 64), (size_t)(sl.groups > 1 ? sl.groups * M : 0)) * N;
+}
+
+int gemm_split(int M, int N, int K) {
+    const Slices sl = slices_of(N, K);
+    return sl.n > 1 ? split_of(M, N, K, sl) : WHOLE;
 }
 
 int launch_panel_pack(int quant, int N, int K, const void* q, const float* s, void* qp, float* sp, hipStream_t st) {

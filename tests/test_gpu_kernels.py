@@ -185,13 +185,36 @@ def test_gemm_rows_independent_of_m(torch_cuda, K, oracle, quant):
     (5760, 1152, (193, 129, 128, 5)),    # two slices, the most panels that have any
     (4096, 1664, (512, 193, 192, 31)),   # slices of 5, 5 and 3: run by one block, and split over blocks
     (4096, 2176, (512, 257, 160, 7)),    # four slices, the last short, in two groups: one block, by slice
-    (2050, 4096, (511, 300, 65)),        # eight slices in two groups, ragged panels: by group, by slice
+    (2050, 4096, (511, 300, 65)),        # eight slices in two groups, ragged panels: one block, by slice
     (13, 512, (65, 2)), (256, 768, (300,)), (136, 4096, (512, 40, 3))])
 def test_gemm_block_shapes(torch_cuda, K, oracle, quant, n, k, rows):
-    """Every block shape and slice form of the prefill GEMM, at the edges of their ranges: against
-    float64 products (1e-5 of the sum of |terms|: 32-bit sums of up to 52 exact block results), and
-    bitwise the same rows in all of them."""
-    torch = torch_cuda
+    """Block shapes and slice forms of the prefill GEMM, at the edges of their ranges (a block per group of
+    slices: test_gemm_by_group): against float64 products (1e-5 of the sum of |terms|: 32-bit sums of up to
+    52 exact block results), and bitwise the same rows in all of them."""
+    _check_gemm_rows(torch_cuda, K, oracle, quant, n, k, rows)
+
+
+# a block per group of slices (2), beside a block per slice (1) and one for all of K (0)
+@pytest.mark.parametrize("quant", [0, 1])
+@pytest.mark.parametrize("n,k,rows,forms", [
+    (4096, 12288, (512, 193, 192, 31), (2, 2, 1, 1)),  # eight slices, four a group: the 9B down product
+    (4109, 2944, (512, 385, 257, 65), (2, 2, 0, 1)),   # slices of 5 x 128 elements, the last of 3; ragged panels
+    (2061, 8192, (480, 384, 300, 7), (2, 2, 1, 1)),    # eight slices, ragged panels
+    (4096, 2176, (512, 192), (0, 1))])                 # too short for it: one block
+def test_gemm_by_group(torch_cuda, K, oracle, quant, n, k, rows, forms):
+    """The form that adds groups of slices: against float64 products (a slice has at most 48 exact block results,
+    a group 4 slices) and bitwise the other forms' rows."""
+    import ctypes
+
+    import snl
+
+    split = getattr(snl.lib(), "_ZN3snl10gemm_splitEiii")  # snl::gemm_split(int M, int N, int K)
+    split.restype = ctypes.c_int
+    assert tuple(split(m, n, k) for m in rows) == forms
+    _check_gemm_rows(torch_cuda, K, oracle, quant, n, k, rows)
+
+
+def _check_gemm_rows(torch, K, oracle, quant, n, k, rows):
     print(f"gemm shapes quant={quant} n={n} k={k} rows={rows}", flush=True)
     q, s, x = _gemv_case(oracle, quant, n, k, rows[0], seed=3 * n + k)
     dq, ds, dx = _dev(torch, q), _dev(torch, s), _dev(torch, x)
