@@ -279,10 +279,13 @@ size_t snl_buffer_size(const snl_engine* e, int id);
 /* ---- kernel-level entry points (device pointers; `stream` is a hipStream_t or NULL) ------ */
 
 /* y[m*y_stride + n] = sum_k x[m*x_stride + k] * W[n, k], M in 1..4 (matmul.wgsl matvec1/2).
- * wq/ws: reference layout quants [N, K] (Q8) or [N, K/2] (Q4), f32 scales [N, K/32].  When
- * K % 128 == 0 the call packs W into the engine's tile order in a staging buffer the library
- * keeps, runs the matrix-core kernel and returns after it has finished on `stream`; other
- * shapes run the vector-ALU kernel on W as given. */
+ * wq/ws: reference layout quants [N, K] (Q8) or [N, K/2] (Q4), f32 scales [N, K/32].  x_stride is
+ * a multiple of 4.  Shapes of the engine's kernel (K % 128 == 0, rows that fit its LDS: K <= 4096 for
+ * M = 3 or 4, 17792 for M = 2) need x on a 16-byte boundary (else SNL_EARG) and return after their work has finished on `stream`: Q8 with
+ * K >= 1024 and wq on a 16-byte boundary is read as given by the vector-ALU kernels, Q4, shorter
+ * rows and other wq are packed into the engine's tile order in a staging buffer the library keeps
+ * and run the matrix-core kernel.  Other shapes run the vector-ALU kernels on W as given, and the
+ * call returns when they are queued. */
 int snl_gemv(int quant, const void* wq, const float* ws, const float* x, float* y, int M, int N, int K,
              int x_stride, int y_stride, void* stream);
 

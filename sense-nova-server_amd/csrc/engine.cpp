@@ -2066,14 +2066,15 @@ int snl_gemv(int quant, const void* wq, const float* ws, const float* x, float* 
     g.K = K;
     g.epi = GEMV_STORE;
     // A Q8 matrix is read where it lies (gemv.hip): packing it into the tile order of the engine's kernel
-    // for one product cost more than the product (2 rows, us a call packed / direct: 12352 x 4096 56 /
-    // 30, 24576 x 4096 87 / 38, 4096 x 12288 56 / 38), with less rounding (1.25e-7 -> 9.6e-8 of the
-    // result, 1.24e-7 -> 1.09e-7 at K = 12288).  The engine's kernel keeps rows shorter than 1024, where a
-    // call is mostly its launch and wait and exact block sums round less (K = 256: 7.8e-8 against 8.2e-8),
-    // and Q4, with the engine's rounding (its -8 x block sum correction, 2e-6 of a result against 1e-7);
-    // also quants that 16-byte loads cannot read.  These are packed into a staging buffer, held under the
-    // lock until the call has finished on the stream.  Shapes of the engine's kernel return when their
-    // work is done, the others when it is queued.
+    // for one product costs more than the product (2 rows, us a call packed / direct: 12352 x 4096 58 / 31,
+    // 24576 x 4096 91 / 37, 4096 x 12288 57 / 37, 4096 x 2048 28 / 19, 256 x 1024 25 / 18).  Its error from K =
+    // 4096 on is smaller too (1.26e-7 -> 9.5e-8 of the result, 12352 x 4096), at 1024 and 2048 the same within
+    // 5%.  The engine's kernel keeps rows shorter than 1024, where its exact block sums round a little less (K =
+    // 256: 7.8e-8 against 8.2e-8), although the direct one would be faster (1544 x 256 18 us a call against 24);
+    // Q4, so that a call gives the engine's own results (its -8 x block sum correction, 1e-6 to 8e-6 of a result
+    // where reading in place would round to 1e-7, and faster); and quants that 16-byte loads cannot read.
+    // These are packed into a staging buffer, held under the lock until the call has finished on the stream.
+    // Shapes of the engine's kernel return when their work is done, the others when it is queued.
     static uint8_t* pq = nullptr;
     static float* ps = nullptr;
     static size_t cap_q = 0, cap_s = 0;
