@@ -467,8 +467,9 @@ def test_model_without_attention_heads(snl_mod, oracle):
 
 @pytest.mark.parametrize("prefix,rows", [(125, 3), (126, 3), (250, 17), (251, 16), (623, 33), (100, 512)])
 def test_prefill_attention_key_parts(snl_mod, prefix, rows):
-    """A prefill pass over cached keys splits them into parts of at least 128 keys; at the parts'
-    edges it gives the logits of the decode kernels (two tokens a pass) within the tolerance."""
+    """A prefill pass over cached keys splits them into parts; at the parts' edges it gives the logits of the
+    decode kernels (two tokens a pass) within 2e-4 of the largest, four times what the other order of every
+    layer's sums was seen to leave (4.6e-5)."""
     cfg = snl_mod.tiny_config()
     n = prefix + rows
     e = snl_mod.Engine(cfg, seed=31, quant=0, ctx=n)
@@ -480,7 +481,7 @@ def test_prefill_attention_key_parts(snl_mod, prefix, rows):
         e.reset()
         for i in range(0, n, 2):
             lg_b, _ = e.forward(prompt[i:i + 2], pos[i:i + 2], logit_rows=len(prompt[i:i + 2]) if i + 2 >= n else 0)
-        assert np.abs(lg_a[-1] - lg_b[-1]).max() / np.abs(lg_b).max() < 1e-3
+        assert np.abs(lg_a[-1] - lg_b[-1]).max() / np.abs(lg_b).max() < 2e-4
     finally:
         e.close()
 
@@ -555,8 +556,9 @@ def test_prefill_cut_at_blocks_of_16(snl_mod, quant):
 @pytest.mark.parametrize("rows", [3, 15, 16, 17, 32, 33, 49])
 def test_prefill_recurrence_blocks(snl_mod, rows):
     """The DeltaNet recurrence of a prefill pass takes 16 tokens at a time, the last block part full:
-    its state and convolution state equal the decode kernels' (one token at a time) within the
-    rounding of 32-bit sums over the tokens, from a state that is not zero."""
+    its state and convolution state equal the decode kernels' (one token at a time), from a state that is not
+    zero, within 3e-4 of the largest: four times what the rounding of all products and layers before it was
+    seen to leave in Q4 (7.2e-5).  The recurrence by itself: test_recurrence_against_64_bits."""
     cfg = snl_mod.tiny_config()
     e = snl_mod.Engine(cfg, seed=37, quant=1, ctx=128)
     try:
@@ -570,9 +572,9 @@ def test_prefill_recurrence_blocks(snl_mod, rows):
         for i in range(40, 40 + rows):
             lg_b, _ = e.forward(prompt[i:i + 1], pos[i:i + 1], logit_rows=1)
         st_b, cv_b = e.buffer(3), e.buffer(4)
-        assert np.abs(st_a - st_b).max() / np.abs(st_b).max() < 1e-3
-        assert np.abs(cv_a - cv_b).max() / np.abs(cv_b).max() < 1e-3
-        assert np.abs(lg_a - lg_b).max() / np.abs(lg_b).max() < 1e-3
+        assert np.abs(st_a - st_b).max() / np.abs(st_b).max() < 3e-4
+        assert np.abs(cv_a - cv_b).max() / np.abs(cv_b).max() < 3e-4
+        assert np.abs(lg_a - lg_b).max() / np.abs(lg_b).max() < 3e-4
     finally:
         e.close()
 
