@@ -19,7 +19,7 @@
 //           16+4g..16+4g+3, the same order in the V^T fragment), A = 16 dims x those keys.
 //
 // A query's keys are summed the same way whatever shares its pass: every leaf of 256 keys (128 within the
-// cache's first 512) from zero, the leaves of 1024 keys to a node, two nodes to a top and the tops one
+// cache's first 1024) from zero, the leaves of 1024 keys to a node, two nodes to a top and the tops one
 // after the other, each time merged in order (merge()).  A part is a leaf, a node or a top (part_level),
 // so a block merges what lies inside its part and pf_combine_kernel the rest, by the same steps; a leaf
 // past a query's position weighs 0 and changes nothing.  Each part leaves (unnormalised output, running max,
@@ -41,9 +41,10 @@ namespace {
 
 constexpr int HD = 256, G = 4;
 constexpr int QTILE = 16, KB = 32;
-// Keys summed from zero, and merged.  The first 512 keys have shorter leaves, for the short contexts whose
-// blocks are few: 45 rows over 260 keys 32 us a launch in leaves of 256, 25 in leaves of 128.
-constexpr int LEAF = 256, FINE = 128, FINE_KEYS = 512, NODE = 1024, TOP = 2 * NODE;
+// Keys summed from zero, and merged.  The first 1024 keys have shorter leaves, for the short contexts whose
+// blocks are few: 45 rows over 260 keys 32 us a call in leaves of 256, 25 in leaves of 128, over 1045 keys 35
+// and 29.  Throughout they would double the merges of long parts (512 rows over 12800 keys 355 us, 381).
+constexpr int LEAF = 256, FINE = 128, FINE_KEYS = 1024, NODE = 1024, TOP = 2 * NODE;
 constexpr int kNodeLeaves = NODE / LEAF, kFirstLeaves = kNodeLeaves + FINE_KEYS / FINE - FINE_KEYS / LEAF;
 constexpr int PSTRIDE = HD + 4;  // floats of a part's partial: output, running max, sum (16-byte rows)
 constexpr int KROW = HD + 8;  // K tile row (halfs): 528 bytes keeps the 16 rows of a read on distinct banks
@@ -405,15 +406,16 @@ static int cdiv(int a, int b) { return (a + b - 1) / b; }
 // The level of the parts of a pass over `keys` keys.  A step of 32 keys is a chain of loads, LDS and dependent
 // MFMAs that one block alone takes 3.3 us for, so few blocks of many steps leave the chip idle (two fit a CU);
 // past two rounds of leaves their partials cost more than longer blocks do.  us a call in parts of a leaf /
-// node / top, 16 heads: 512 rows over 2048 keys 98 / 101 / 175 (1024 blocks of a leaf), 4600 200 / 157 / 176,
+// node / top, 16 heads, leaves of 256: 512 rows over 2048 keys 98 / 101 / 175 (1024 blocks of a leaf), 4600 200 / 157 / 176,
 // 12800 495 / 342 / 355 (1664 blocks of a node), 32768 1336 / 837 / 796; 100 rows over 7000 keys 74 / 88 / 156,
 // 9500 102 / 94 / 157; 45 rows over 12800 keys 76 / 88 / 156.
 // Parts of any length, cut by the blocks that a pass gives, were faster where rows are many (512 rows over
-// 1000 keys 69 us, 72 so; 12800 314 and 345; 45 rows over 1045 30 and 35) and slower where they are few (3 over
-// 12800 74 and 48), but a token's sums then changed with the tokens that shared its pass.
+// 1045 keys 69 us, 72 so; 2048 91 and 104; 12800 322 and 352) and slower where they are few (3 over 12800 keys
+// 74 and 48) or the keys (512 rows over 520 55 and 49, 200 over 1045 47 and 42), but a token's sums then changed
+// with the tokens that shared its pass.
 // A launch takes as many query tiles as keep its partials within kMaxBlocks blocks' (136 MB, 16 heads at any
 // context).
-constexpr int kLeafBlocks = 1024, kMaxBlocks = 2048;
+constexpr int kLeafBlocks = 1280, kMaxBlocks = 2048;
 static int part_level(int tiles, int n_kv, int keys) {
     if (keys <= FINE || n_kv * tiles * part_count(0, keys) <= kLeafBlocks) return 0;
     return keys <= NODE || n_kv * tiles * part_count(1, keys) <= kMaxBlocks ? 1 : 2;

@@ -488,8 +488,8 @@ def test_prefill_attention_key_parts(snl_mod, prefix, rows):
 
 @pytest.fixture(scope="module")
 def attention_only(snl_mod):
-    """Engines of two attention layers: 1 KV head (the key parts of a pass are 128 and 256 keys long, from 7936
-    keys of 512 rows on 1024) and 16 KV heads (512 rows: up to 256 keys, then 1024 a part, from 4096 on 2048,
+    """Engines of two attention layers: 1 KV head (the key parts of a pass are 128 and 256 keys long, past
+    9216 keys of 512 rows 1024) and 16 KV heads (512 rows: up to 256 keys, then 1024 a part, from 4096 on 2048,
     and past 8192 keys two launches)."""
     import dataclasses
 
@@ -507,7 +507,7 @@ def attention_only(snl_mod):
     (1, 270, [(270,), (3, 267), (255, 15), (128, 128, 14)]),
     (1, 1045, [(1000, 45), (1003, 42), (300, 700, 45), (512, 530, 3)]),
     (1, 9750, [(9216, 534), (9217, 17, 516), (9100, 300, 47, 303)]),
-    (1, 523, [(523,), (509, 14), (512, 8, 3), (384, 139)]),
+    (1, 1291, [(1291,), (1021, 270), (1024, 256, 11), (512, 515, 264)]),
     (16, 8300, [(8300,), tuple([48] * 172 + [44]), (1024, 513, 511, 3000, 3252)])])
 def test_prefill_token_independent_of_its_pass(attention_only, n_kv, n, splits):
     """A token's results do not depend on which tokens share its pass: the last two logits rows of a prompt (which
